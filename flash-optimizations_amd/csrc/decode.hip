@@ -95,10 +95,11 @@ struct DecodeArgs {
   int64_t freq_rows;
   const float* inv_freq;   // position mode: [32] inverse frequencies (nullptr: identity)
   float scale_log2;
-  int64_t q_len;
+  uint64_t q_len_magic;  // ceil(2^32 / q_len): token t < 2^16 is of request t * q_len_magic >> 32
   int64_t heads;
   int chunk;       // records per split (multiple of 32)
   int splits;      // splits of this list (workgroups along x)
+  uint32_t splits_magic;  // ceil(2^16 / splits): x / splits = x * splits_magic >> 16 for x < 2^10
   int ws_splits;   // partial slots per row in the workspace; 0: finalise in place
   int ws_base;     // slot of this list's split 0
   uint16_t* out;
@@ -205,7 +206,8 @@ constexpr int kPcKPitch = kHeadDim + 16;   // BF16 per K row (1056 B: rows 8 ban
 // group (one even, one odd chunk, 4 rows) cover 32 distinct banks.
 constexpr int kPcOddAt = 264;
 __device__ __forceinline__ constexpr int kchunk(int q) { return (q >> 1) * 8 + (q & 1) * kPcOddAt; }
-constexpr int kPcMaxChunk = 512;           // records per split
+constexpr int kPcMaxChunk = 512;           // record slots of a split's table
+constexpr int kBtCache = 1024;             // block-table columns looked up in LDS
 // instruction classes of __builtin_amdgcn_sched_group_barrier
 constexpr int kSchedMfma = 0x008;
 constexpr int kSchedDsRead = 0x100;
@@ -290,6 +292,12 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
   auto& aux_tab = sm->aux_tab;
   auto& mrg = sm->mrg;
 
+  // every argument of the set-up requested at once (the compiler would load
+  // them in three dependent groups, each at its first use)
+  asm volatile("" ::"s"(a.q), "s"(a.pool), "s"(a.pool_pages), "s"(a.pool_rows), "s"(a.block_table),
+               "s"(a.bt_stride), "s"(a.max_blocks), "s"(a.seqlens), "s"(a.indices), "s"(a.topk),
+               "s"(a.topk_length), "s"(a.freqs), "s"(a.freq_rows), "s"(a.inv_freq),
+               "s"(a.q_len_magic), "s"(a.heads), "s"(a.splits), "s"(a.splits_magic));
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   // Role index of this wave. A workgroup's waves fill SIMDs 0..3 in order
@@ -311,63 +319,34 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
   // -> 28.0 us (positions). Long splits (B=128 x next-n 2 94 -> 98-102 us)
   // and single-stage splits (B=1) keep the default placement.
   const int wv_hw = uniform(tid >> 6);
-  const bool several = (a.topk + kPcStage - 1) / kPcStage > (int64_t)a.splits;
+  const bool several = ((int)a.topk + kPcStage - 1) / kPcStage > a.splits;
   const bool remap = !kPacked && kHG == 1 && several;
   const bool tail_remap = kHelp && kPacked && !kLong && several;
   const int wv = remap ? (wv_hw == 2 ? 0 : wv_hw == 3 ? 1 : wv_hw < 2 ? wv_hw + 2 : wv_hw)
                  : tail_remap && wv_hw >= 4 ? (wv_hw ^ 2)
                                             : wv_hw;
   const int64_t t = blockIdx.y;
+  const int splits = a.splits, topk = (int)a.topk;
   const int64_t head_wg = (int64_t)blockIdx.z * 16 * kHG;
   // a consumer's 16 heads (consumers 2 hg and 2 hg + 1 serve group hg)
   const int64_t head0 = head_wg + (wv < kPcConsumers ? 16 * (wv >> 1) : 0);
-  const int64_t b = t / a.q_len;
+  const int64_t b = (int64_t)(((uint64_t)t * a.q_len_magic) >> 32);
 
-  int64_t len = a.topk;
-  if (a.topk_length) {
-    const int64_t l = a.topk_length[t];
-    len = l < 0 ? 0 : (l < a.topk ? l : a.topk);
-  }
-  // this token's valid entries in whole stages, spread evenly over the splits
-  // (at most a.chunk each, since len <= topk): a short list finishes early in
-  // every split instead of emptying the last ones
-  const int64_t len_stages = (len + kPcStage - 1) / kPcStage;
-  const int64_t chunk = ((len_stages + a.splits - 1) / a.splits) * kPcStage;
-  const int64_t k0 = (int64_t)split * chunk;
-  const int64_t k1 = k0 + chunk < len ? k0 + chunk : len;
-  const int n = k1 > k0 ? (int)(k1 - k0) : 0;
-  const int stages = (n + kPcStage - 1) / kPcStage;
-  const int64_t seqlen = a.seqlens ? a.seqlens[b] : INT64_MAX;
+  // Stage j of this split is stage j * splits + split of the list: where a
+  // record sits does not depend on the list's valid length, so the top-k
+  // entries are requested together with the length, and a short list still
+  // spreads evenly over the splits (to within one stage).
+  auto list_pos = [&](int i) {
+    return ((i >> 5) * splits + split) * kPcStage + (i & (kPcStage - 1));
+  };
+  static_assert(kPcStage == 32, "list_pos");
 
-  // Consumers hold Q of the 16 heads as the B operand of S^T = K Q^T:
-  // qf[ks] = Q[head lane % 16][32 ks + 8 (lane / 16) .. +7]
-  bf16x8 qf[16];
-  if (wv < kPcConsumers) {
-    const uint16_t* qh = a.q + (t * a.heads + head0 + (lane & 15)) * kHeadDim + 8 * (lane >> 4);
-#pragma unroll
-    for (int ks = 0; ks < 16; ++ks) qf[ks] = __builtin_bit_cast(bf16x8, *(const u32x4*)(qh + 32 * ks));
-  }
-
-  // ---- setup: selectors, record metadata ----
-  if (kPacked && tid < 256) {
-    const uint32_t e = tid;
-    uint32_t r = 0;
-    uint64_t sel = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const bool kept = (e >> (7 - i)) & 1u;
-      sel |= (uint64_t)(kept ? r : 0x0cu) << (8 * i);
-      r += kept ? 1u : 0u;
-    }
-    sel_tab[e] = sel;
-  }
+  // ---- setup: record metadata, selectors ----
   const uint64_t stand_in = (uint64_t)a.q | 1u;
   const bool paged = a.block_table != nullptr;
-  // whether logical record r of request b has a block-table entry to read
-  auto in_table = [&](int64_t r) { return r >= 0 && r < seqlen && (r >> 6) < a.max_blocks; };
   // table entry of record slot i from its top-k entry r (< 0: none) and, for
   // a paged pool, its block-table entry pv (meaningful only when in_table(r))
-  auto put_entry = [&](int i, int64_t r, int64_t pv) {
+  auto put_entry = [&](int i, int64_t r, int64_t pv, auto in_table) {
     bool ok;
     int64_t page;
     if (paged) {  // logical record of request b
@@ -393,31 +372,96 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
     if (kPacked && kPos) aux_tab[slot] = f2u(ok ? (float)(4 * r) : 0.0f);
     else if (kPacked) aux_tab[slot] = a.freqs ? (uint64_t)(a.freqs + (ok ? r : 0) * 4 * 64) : (uint64_t)a.q;
   };
-  // the first kPcMaxChunk slots, read directly by all threads
-  constexpr int kEntries = (kPcMaxChunk + kPcThreads - 1) / kPcThreads;  // per thread
-  auto build_table = [&]() {
-    int64_t r[kEntries], pv[kEntries];
+  // The first kPcMaxChunk slots, by all waves but the consumers. The list's
+  // length, its top-k entries and, for tables of at most kBtCache columns, the
+  // request's block-table row are requested side by side, every load
+  // unconditional (clamped to what is there) so that no wait comes between
+  // two; the row is then looked up in LDS (in the K ring, idle here). The
+  // records' addresses are one memory round trip away from the arguments
+  // instead of four (length, sequence length, top-k entries, block table).
+  // Wider tables look their entries up in memory, one round trip more.
+  constexpr int kBuilders = kPcThreads - 64 * kPcConsumers;
+  constexpr int kEntries = (kPcMaxChunk + kBuilders - 1) / kBuilders;  // per thread
+  constexpr int kBtLoads = (kBtCache + kBuilders - 1) / kBuilders;
+  const int btid = (wv - kPcConsumers) * 64 + lane;
+  const bool builder = wv >= kPcConsumers;
+  const int32_t* const none = (const int32_t*)a.q;
+  const bool bt_cached = paged && a.max_blocks <= kBtCache;
+  int32_t* const bt_lds = (int32_t*)&ktile[0][0];
+  static_assert(sizeof(ktile) >= kBtLoads * kBuilders * sizeof(int32_t), "row in the K ring");
+  // (scalar loads)
+  using const_i32 = __attribute__((address_space(4))) const int32_t;
+  const int len_raw = *(const_i32*)(uintptr_t)(a.topk_length ? a.topk_length + t : none);
+  const int seq_raw = *(const_i32*)(uintptr_t)(a.seqlens ? a.seqlens + b : none);
+  int32_t r0[kEntries], bv[kBtLoads];
+  auto load_entries = [&]() {
+    const int32_t* const list = topk > 0 ? a.indices + t * topk : none;
+    const uint32_t last = topk > 0 ? topk - 1 : 0;
 #pragma unroll
-    for (int j = 0; j < kEntries; ++j) {  // top-k entries
-      const int i = tid + j * kPcThreads;
-      r[j] = -1;
-      pv[j] = 0;
-      if (i < kPcMaxChunk && i < n) r[j] = a.indices[t * a.topk + k0 + i];
-    }
-    // then every block-table entry, by unconditional loads (Q's first word
-    // stands in where there is none): the compiler waits for a load made inside
-    // a branch before the next one, which would serialise a thread's entries
+    for (int j = 0; j < kEntries; ++j) r0[j] = list[min((uint32_t)list_pos(btid + j * kBuilders), last)];
+    const int32_t* const row = bt_cached ? a.block_table + b * a.bt_stride : none;
+    const uint32_t last_col = bt_cached && a.max_blocks > 0 ? (uint32_t)a.max_blocks - 1 : 0;
 #pragma unroll
-    for (int j = 0; j < kEntries; ++j) {
-      const bool has = paged && in_table(r[j]);
-      const int32_t* src = has ? a.block_table + (b * a.bt_stride + (r[j] >> 6)) : (const int32_t*)a.q;
-      const int32_t v = *src;
-      pv[j] = has ? v : 0;
+    for (int j = 0; j < kBtLoads; ++j) bv[j] = row[min((uint32_t)(btid + j * kBuilders), last_col)];
+  };
+  // Consumers hold Q of the 16 heads as the B operand of S^T = K Q^T:
+  // qf[ks] = Q[head lane % 16][32 ks + 8 (lane / 16) .. +7]
+  bf16x8 qf[16];
+  if (builder) {
+    load_entries();
+  } else {
+    const uint16_t* qh = a.q + (t * a.heads + head0 + (lane & 15)) * kHeadDim + 8 * (lane >> 4);
+#pragma unroll
+    for (int ks = 0; ks < 16; ++ks) qf[ks] = __builtin_bit_cast(bf16x8, *(const u32x4*)(qh + 32 * ks));
+  }
+  if (kPacked && builder && btid < 256) {  // while the loads are in flight
+    const uint32_t e = btid;
+    uint32_t r = 0;
+    uint64_t sel = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const bool kept = (e >> (7 - i)) & 1u;
+      sel |= (uint64_t)(kept ? r : 0x0cu) << (8 * i);
+      r += kept ? 1u : 0u;
     }
+    sel_tab[e] = sel;
+  }
+  // valid entries of this token's list, and this split's stages of them
+  const int len = !a.topk_length || len_raw > topk ? topk : max(len_raw, 0);
+  const int len_stages = (len + kPcStage - 1) / kPcStage;
+  const int stages = len_stages > split
+                         ? (int)(((uint32_t)(len_stages - 1 - split) * a.splits_magic) >> 16) + 1
+                         : 0;
+  const int64_t seqlen = a.seqlens ? seq_raw : INT64_MAX;
+  // whether logical record r of request b has a block-table entry to read
+  auto in_table = [&](int64_t r) { return r >= 0 && r < seqlen && (r >> 6) < a.max_blocks; };
+  auto make_entries = [&]() {
+    int32_t pv[kEntries];
+    if (bt_cached) {
+      if (builder) {
+#pragma unroll
+        for (int j = 0; j < kBtLoads; ++j) bt_lds[btid + j * kBuilders] = bv[j];
+      }
+      block_sync_lds();  // the row is in LDS
+    }
+    if (!builder) return;
 #pragma unroll
     for (int j = 0; j < kEntries; ++j)
-      if (tid + j * kPcThreads < kPcMaxChunk) put_entry(tid + j * kPcThreads, r[j], pv[j]);
+      if (bt_cached)
+        pv[j] = bt_lds[in_table(r0[j]) ? r0[j] >> 6 : 0];
+      else
+        pv[j] = *(paged && in_table(r0[j]) ? a.block_table + (b * a.bt_stride + (r0[j] >> 6)) : none);
+#pragma unroll
+    for (int j = 0; j < kEntries; ++j) {
+      const int i = btid + j * kBuilders;
+      if (i < kPcMaxChunk) put_entry(i, list_pos(i) < len ? r0[j] : -1, pv[j], in_table);
+    }
   };
+  auto build_table = [&]() {
+    if (builder) load_entries();
+    make_entries();
+  };
+
   // position mode: theta of the four RoPE pairs a producer lane rotates
   // (lane / 8 = j: pairs 4 j .. 4 j + 3; zero, the identity, without inverse
   // frequencies), loaded with the table and retired before the stage loop (the
@@ -435,9 +479,11 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
       theta = *(const f32x4*)(a.inv_freq + 4 * (lane >> 3));
     }
   }
-  build_table();
-  wait_vm();
-  __syncthreads();
+  make_entries();
+  // (the consumers' Q may still be in flight; the other waves' waits below
+  // count their loads from none outstanding)
+  if (builder) wait_vm();
+  block_sync_lds();
   if constexpr (kPos) asm volatile("" : "+v"(theta), "+v"(theta2));
 
   // Splits of more than kPcMaxChunk records: consumer 0 refills the table
@@ -457,13 +503,13 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
     int q = s + 4;
     if (q >= kRingStages && q < stages && ln < kPcStage) {
       const int i = q * kPcStage + ln;
-      const int64_t r = i < n ? (int64_t)sm->idx_ring[q % 3][ln] : -1;
-      put_entry(i, r, sm->bt_ring[q % 3][ln]);
+      const int64_t r = list_pos(i) < len ? (int64_t)sm->idx_ring[q % 3][ln] : -1;
+      put_entry(i, r, sm->bt_ring[q % 3][ln], in_table);
     }
     q = s + 5;
     if (q >= kRingStages && q < stages) {
       const int i = q * kPcStage + ln;
-      const int64_t r = ln < kPcStage && i < n ? (int64_t)sm->idx_ring[q % 3][ln] : -1;
+      const int64_t r = ln < kPcStage && list_pos(i) < len ? (int64_t)sm->idx_ring[q % 3][ln] : -1;
       const int32_t* src = paged && in_table(r) ? a.block_table + (b * a.bt_stride + (r >> 6))
                                                 : (const int32_t*)a.q;
       dma4_opaque(src, lds_addr(&sm->bt_ring[q % 3][0]));
@@ -471,8 +517,8 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
     q = s + 6;
     if (q >= kRingStages && q < stages) {
       const int i = q * kPcStage + ln;
-      const int32_t* src = ln < kPcStage && i < n ? a.indices + (t * a.topk + k0 + i)
-                                                  : (const int32_t*)a.q;
+      const int32_t* src = ln < kPcStage && list_pos(i) < len ? a.indices + (t * a.topk + list_pos(i))
+                                                              : (const int32_t*)a.q;
       dma4_opaque(src, lds_addr(&sm->idx_ring[q % 3][0]));
     }
   };
@@ -966,6 +1012,7 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
   // Consumer c owns output coordinates 256 c .. 256 c + 255 of the 16 heads.
   // Both consumers score every tile, so their softmax state (reference, sum)
   // is identical and each finalises its half of O on its own.
+  wait_vm();  // Q
   const int g = lane >> 4, col = lane & 15;
   const int half = wv & 1;  // 0 or 1
   f32x4 o[16];          // O[head 4g + i][256 half + 16 nt + col]
@@ -1485,10 +1532,11 @@ int launch_decode(const uint16_t* q, int64_t batch, int64_t q_len, int64_t heads
   // (theta = 0, the identity, with neither)
   const bool pos = kPacked && (inv_freq || !freqs);
   a.scale_log2 = scale * kLog2e;
-  a.q_len = q_len;
+  a.q_len_magic = (((uint64_t)1 << 32) + q_len - 1) / q_len;
   a.heads = heads;
   a.chunk = plan.chunk;
   a.splits = plan.splits;
+  a.splits_magic = (65536 + plan.splits - 1) / plan.splits;
   a.ws_splits = slots > 1 ? (int)slots : 0;
   a.ws_base = 0;
   a.out = out;
@@ -1521,6 +1569,7 @@ int launch_decode(const uint16_t* q, int64_t batch, int64_t q_len, int64_t heads
     b.inv_freq = nullptr;
     b.chunk = kPcMaxChunk;
     b.splits = 1;
+    b.splits_magic = 65536;
     b.ws_base = plan.splits;
     const dim3 grid((unsigned)slots, (unsigned)tokens, zblocks);
     const JointKernel kern = lng ? joint_kernel<kPacked, true>(src.planes(), hg, pos)

@@ -488,3 +488,29 @@ def test_native_decode_pool_beyond_4gib_offsets():
     per_row_check(out.float().cpu().numpy(), ref, lse.cpu().numpy(), ref_lse)
     del pool
     torch.cuda.empty_cache()
+
+
+# ---- block-table width: rows looked up in LDS up to 1,024 columns -------------------------
+
+@pytest.mark.parametrize("packed", [True, False], ids=["direct", "native"])
+def test_decode_block_table_width_and_interleaved_stages(packed):
+    """Requests of 1 to 700 records, three query tokens each (a token's request
+    by the q_len reciprocal), list lengths that end in every position of the
+    splits' interleaved stages. The table as it is, padded to 1,024 columns
+    (looked up in LDS) and to 1,025 (looked up in memory): the same bits, and
+    within tolerance of the oracle."""
+    banner(f"decode block-table width packed={packed}")
+    ctx = [700, 1, 64, 65, 333]
+    c = build_decode_case(ctx, q_len=3, heads=16, topk=417, seed=487, packed=packed)
+    lens = c["lens"].reshape(-1)
+    for t, n in ((1, 0), (2, 31), (12, 32), (13, 33), (14, 257)):
+        lens[t] = min(n, lens[t])
+    out, lse = run_decode(c)
+    ref, ref_lse = oracle_decode(c)
+    per_row_check(out, ref, lse, ref_lse)
+    table = c["table"]
+    for width in (1024, 1025):
+        c["table"] = np.full((len(ctx), width), -1, np.int32)
+        c["table"][:, :table.shape[1]] = table
+        got, got_lse = run_decode(c)
+        assert np.array_equal(got, out) and np.array_equal(got_lse, lse)
