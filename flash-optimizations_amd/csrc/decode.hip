@@ -266,6 +266,23 @@ __device__ __forceinline__ float max_over_rows(float x) {
   return fmaxf(u2f(r[0]), u2f(r[1]));
 }
 
+// Sum of x over the same lanes.
+__device__ __forceinline__ float sum_over_rows(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false,
+                                                  false);
+  x = u2f(r[0]) + u2f(r[1]);
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
+                                                  false);
+  return u2f(h[0]) + u2f(h[1]);
+}
+
+// Order of a split partial's 512 floats: coordinate 64 u + 16 q + c (u < 8, q <
+// 4, c < 16) is at 64 u + 4 c + q, so the 16-coordinate stride at which a
+// consumer lane holds its coordinates becomes four runs of four.
+__device__ __forceinline__ constexpr int partial_coord(int at) {
+  return (at & ~63) + 16 * (at & 3) + ((at & 63) >> 2);
+}
+
 // One workgroup's share: split `split` of list `a` (a C4 top-k list through
 // the block table, or with a.block_table == nullptr a list of pool slots), for
 // kHG groups of 16 heads: every expanded record serves all of them.
@@ -1114,8 +1131,7 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
     // a split of one stage took its reference from that stage: no overflow,
     // and both roles skip the test's two barriers
     if (stages <= 1) break;
-    m_seen = fmaxf(m_seen, __shfl_xor(m_seen, 16, 64));
-    m_seen = fmaxf(m_seen, __shfl_xor(m_seen, 32, 64));
+    m_seen = max_over_rows(m_seen);
     if (lane < 16) {
       mrg[wv][0][lane] = m_ref;
       mrg[wv][1][lane] = m_seen;
@@ -1134,45 +1150,53 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
   }
 
   // ---- finalise this consumer's half of O ----
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);  // sum of the weights of head col against m_ref
+  l_run = sum_over_rows(l_run);  // sum of the weights of head col against m_ref
   const float mm = m_ref;
-  float factor_h, lse_h;
-  if (a.ws_splits == 0) {
-    const float sink2 = a.sink ? a.sink[head0 + col] * kLog2e : -INFINITY;
-    const float mz = fmaxf(mm, sink2);
-    factor_h = 0.0f;
-    lse_h = -INFINITY;
-    if (mz != -INFINITY) {
-      const float em = mm == -INFINITY ? 0.0f : exp2f(mm - mz);
-      const float z = l_run * em + exp2f(sink2 - mz);
-      factor_h = em / z;
-      lse_h = (mz + log2f(z)) * kLn2;
-    }
-    if (half == 0 && lane < 16) a.lse[t * a.heads + head0 + col] = lse_h;
-  } else {
-    factor_h = l_run > 0.0f ? 1.0f / l_run : 0.0f;
-    lse_h = l_run > 0.0f ? mm + log2f(l_run) : -INFINITY;
+  // One branch to each of the two ends, each straight-line code with its four
+  // head factors exchanged at once: this code runs once per workgroup, so its
+  // time is instruction fetch and exchange latency.
+  auto head_factors = [&](float factor_h, float (&f)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f[i] = __shfl(factor_h, 4 * g + i, 64);
+  };
+  float f[4];
+  if (a.ws_splits != 0) {
+    head_factors(l_run > 0.0f ? 1.0f / l_run : 0.0f, f);
+    // Partials in partial_coord() order: four 16-byte stores cover a lane's 16
+    // coordinates and a store instruction 256 contiguous bytes of each of its
+    // four rows, where the coordinates' own order would take 16 stores of 4
+    // bytes in 64-byte runs. Streaming stores: the partials are read once, by
+    // the combine.
+    const int64_t slot = (t * a.ws_splits + a.ws_base + split) * a.heads + head0;
+    float* const orow = a.ws_o + (slot + 4 * g) * kHeadDim + 256 * half + 4 * col;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        __builtin_nontemporal_store(f32x4{o[4 * j][i] * f[i], o[4 * j + 1][i] * f[i],
+                                          o[4 * j + 2][i] * f[i], o[4 * j + 3][i] * f[i]},
+                                    (f32x4*)(orow + i * kHeadDim + 64 * j));
     if (half == 0 && lane < 16)
-      a.ws_lse[(t * a.ws_splits + a.ws_base + split) * a.heads + head0 + col] = lse_h;
+      a.ws_lse[slot + col] = l_run > 0.0f ? mm + log2f(l_run) : -INFINITY;
+    return;
   }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int h = 4 * g + i;
-    const float f = __shfl(factor_h, h, 64);
-    if (a.ws_splits == 0) {
-      uint16_t* orow = a.out + (t * a.heads + head0 + h) * kHeadDim + 256 * half + col;
-#pragma unroll
-      for (int nt = 0; nt < 16; ++nt)
-        orow[16 * nt] = __builtin_bit_cast(uint16_t, (__bf16)(o[nt][i] * f));
-    } else {
-      float* orow = a.ws_o + ((t * a.ws_splits + a.ws_base + split) * a.heads + head0 + h) * kHeadDim +
-                    256 * half + col;
-      // streaming stores: the partials are read once, by the combine
-#pragma unroll
-      for (int nt = 0; nt < 16; ++nt) __builtin_nontemporal_store(o[nt][i] * f, orow + 16 * nt);
-    }
+  const float sink2 = a.sink ? a.sink[head0 + col] * kLog2e : -INFINITY;
+  const float mz = fmaxf(mm, sink2);
+  float factor_h = 0.0f, lse_h = -INFINITY;
+  if (mz != -INFINITY) {
+    const float em = mm == -INFINITY ? 0.0f : exp2f(mm - mz);
+    const float z = l_run * em + exp2f(sink2 - mz);
+    factor_h = em / z;
+    lse_h = (mz + log2f(z)) * kLn2;
   }
+  if (half == 0 && lane < 16) a.lse[t * a.heads + head0 + col] = lse_h;
+  head_factors(factor_h, f);
+  uint16_t* const orow = a.out + (t * a.heads + head0 + 4 * g) * kHeadDim + 256 * half + col;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int nt = 0; nt < 16; ++nt)
+      orow[i * kHeadDim + 16 * nt] = __builtin_bit_cast(uint16_t, (__bf16)(o[nt][i] * f[i]));
 }
 
 // kLong: splits may run past kPcMaxChunk records (the table ring refill),
@@ -1278,7 +1302,7 @@ __device__ __forceinline__ float lane_of(float x, int l) {
 }
 
 // Merge split partials with the sink, for many rows: one wave per (token,
-// head) row, lane l owning coordinates 8l..8l+7. The partial loads of up to
+// head) row, lane l owning the coordinates stored at 8l..8l+7. The partial loads of up to
 // kWaveBatch splits are issued together with the split LSEs (lane s holds
 // split s), so a row costs one round trip per kWaveBatch splits.
 constexpr int kWaveBatch = 8;
@@ -1333,14 +1357,17 @@ __global__ __launch_bounds__(256) void combine_wave_kernel(const float* __restri
     r1 = a1 * inv;
     lse_out = (mz + log2f(zt)) * kLn2;
   }
-  *(u32x4*)(out + row * kHeadDim + 8 * lane) =
-      u32x4{bf16_rne(r0[0]) | (bf16_rne(r0[1]) << 16), bf16_rne(r0[2]) | (bf16_rne(r0[3]) << 16),
-            bf16_rne(r1[0]) | (bf16_rne(r1[1]) << 16), bf16_rne(r1[2]) | (bf16_rne(r1[3]) << 16)};
+  // r0[q] and r1[q] are neighbouring coordinates: partial_coord(8 lane + q) and + 1
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    *(uint32_t*)(out + row * kHeadDim + partial_coord(8 * lane + q)) =
+        bf16_rne(r0[q]) | (bf16_rne(r1[q]) << 16);
   if (lane == 0) lse[row] = lse_out;
 }
 
 // Merge split partials with the sink, for few rows (small batches). One
-// workgroup (4 waves) per (token, head, 64-coordinate slice): lane l owns coordinate 64 slice + l; wave w takes
+// workgroup (4 waves) per (token, head, 64-coordinate slice): lane l owns the
+// coordinate stored at 64 slice + l; wave w takes
 // splits w, w + 4, ... (<= 16 each, all loads in flight at once); the four
 // partial sums meet in LDS in a fixed order. The split weights come from every
 // split's LSE, read by every wave (lane s holds split s; splits <= 64).
@@ -1387,7 +1414,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
       r = (part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane]) * inv;
       lse_out = (mz + log2f(zt)) * kLn2;
     }
-    out[row * kHeadDim + 64 * slice + lane] = (uint16_t)bf16_rne(r);
+    out[row * kHeadDim + partial_coord(64 * slice + lane)] = (uint16_t)bf16_rne(r);
     if (lane == 0 && slice == 0) lse[row] = lse_out;
   }
 }
