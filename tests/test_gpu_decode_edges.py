@@ -514,3 +514,19 @@ def test_decode_block_table_width_and_interleaved_stages(packed):
         c["table"][:, :table.shape[1]] = table
         got, got_lse = run_decode(c)
         assert np.array_equal(got, out) and np.array_equal(got_lse, lse)
+
+
+# ---- combine: every count of partials its unrolled loads switch at ------------------------
+
+@pytest.mark.parametrize("topk", [128, 160, 256, 288, 512, 544, 1024, 1056, 2048])
+@pytest.mark.parametrize("tokens", [1, 4])
+def test_decode_combine_split_counts(tokens, topk):
+    """4 to 64 splits of one stage each (one token: the 64-coordinate combine,
+    unrolled for 16, 32 and 64 splits) and the same lists over four tokens with
+    64 heads (the row combine, unrolled for 4 and 8 splits)."""
+    banner(f"decode combine tokens={tokens} topk={topk}")
+    c = build_decode_case([2100] * tokens, q_len=1, heads=16 if tokens == 1 else 64, topk=topk,
+                          seed=491 + topk, packed=True)
+    out, lse = run_decode(c)
+    ref, ref_lse = oracle_decode(c)
+    per_row_check(out, ref, lse, ref_lse)
