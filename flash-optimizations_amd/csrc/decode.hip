@@ -30,8 +30,8 @@
 //     staged rows (in table mode with RoPE rows it loads into registers two
 //     stages ahead), so the producers expand only the 448 other coordinates
 //     and rotate nothing. By default they sit beside the two producers that
-//     have no consumer beside them; on splits of several stages of at most
-//     512 records beside the consumers, the producers paired on the other
+//     have no consumer beside them; on splits of several stages whose record
+//     table is not refilled beside the consumers, the producers paired on the other
 //     two SIMDs (B=64 29.8 -> 27.9 us from positions, 29.9 -> 28.6 us from
 //     the table);
 //   * two consumer waves each own 256 of the 512 output coordinates. Both
@@ -43,8 +43,8 @@
 //     2^64 are far inside FP32/BF16 range; a split whose scores climb higher
 //     is recomputed once against its true max;
 //   * one workgroup barrier per stage hands the ring over: producers fill
-//     stage s while consumers read stage s - 1. On splits of at most 512
-//     records the producers run at a higher wave priority than the consumers
+//     stage s while consumers read stage s - 1. On splits whose record table
+//     is not refilled the producers run at a higher wave priority than the consumers
 //     (with the default placement two SIMDs hold one of each, and the
 //     producers set the stage time).
 // A Packed record (328 B, 8-byte aligned) is fetched as the 21 aligned 16-byte
@@ -206,7 +206,15 @@ constexpr int kPcKPitch = kHeadDim + 16;   // BF16 per K row (1056 B: rows 8 ban
 // group (one even, one odd chunk, 4 rows) cover 32 distinct banks.
 constexpr int kPcOddAt = 264;
 __device__ __forceinline__ constexpr int kchunk(int q) { return (q >> 1) * 8 + (q & 1) * kPcOddAt; }
-constexpr int kPcMaxChunk = 512;           // record slots of a split's table
+constexpr int kPcMaxChunk = 512;           // records of a short split; window rows at most
+// Split lengths, each compiled apart: short (at most 512 records), whole
+// (Packed, at most 2,048: a table of that size, built once; it does not fit
+// beside the Native copy ring) and refilled (beyond: a table of 512 slots that
+// a consumer refills as the split streams). The refill and the wave placement
+// and priorities it forbids cost a quarter of a stage: B=128 x next-n 2 at
+// top-k 2048, one split per token, 95.7 us refilled, 78.8 us whole.
+enum Len { kShort, kWhole, kRefill };
+constexpr int table_slots(Len l) { return l == kWhole ? 2048 : kPcMaxChunk; }
 constexpr int kBtCache = 1024;             // block-table columns looked up in LDS
 // instruction classes of __builtin_amdgcn_sched_group_barrier
 constexpr int kSchedMfma = 0x008;
@@ -229,19 +237,20 @@ struct PcGeo {
 // Shared memory of one workgroup. The kernels declare one byte array of the
 // larger format's size and view it as the format they run, so a kernel that
 // runs either format per workgroup needs no more LDS than the larger one.
-template <bool kPacked>
+template <bool kPacked, Len kLen = kShort>
 struct PcShared {
   using G = PcGeo<kPacked>;
   uint8_t raw[kPcProducers][G::kDepth][G::kBuf];  // copy ring (LDS address 0)
   uint16_t ktile[kPcRing][kT * kPcKPitch];
-  // per record slot of the split, a ring of kPcMaxChunk entries (record i at
-  // i % kPcMaxChunk; splits of more than kPcMaxChunk records refill it as they
+  static constexpr int kTab = table_slots(kLen);
+  // per record slot of the split, a ring of kTab entries (record i at
+  // i % kTab; refilled splits, of more records than that, refill it as they
   // go): pool row address, or (Q address | 1) for an invalid record or a slot
   // past the end (a readable stand-in source, odd so that bit 0 marks it);
   // Packed: RoPE row address (row 0 of the table for an invalid record, Q
   // without a table)
-  uint64_t row_tab[kPcMaxChunk];
-  uint64_t aux_tab[kPacked ? kPcMaxChunk : 1];
+  uint64_t row_tab[kTab];
+  uint32_t aux_tab[kPacked ? kTab : 1];
   // long splits: the records' top-k entries and block-table entries of the
   // next stages, copied in ahead of the table entries made from them
   int32_t idx_ring[3][64];
@@ -253,8 +262,10 @@ struct PcShared {
   alignas(16) uint8_t rope_ring[kPacked ? kPcProducers * 2 * 2 * 1024 : 1];
   float mrg[2 * kPcMaxGroups][2][16];  // consumers' (reference, seen) maxima per head
 };
-constexpr size_t kPcSmemBytes = sizeof(PcShared<true>) > sizeof(PcShared<false>)
-                                    ? sizeof(PcShared<true>) : sizeof(PcShared<false>);
+template <bool kPacked, Len kLen>
+constexpr size_t kJointSmemBytes = sizeof(PcShared<kPacked, kLen>) > sizeof(PcShared<false>)
+                                       ? sizeof(PcShared<kPacked, kLen>) : sizeof(PcShared<false>);
+static_assert(sizeof(PcShared<true, kWhole>) <= 160 * 1024, "LDS of a CU");
 
 // Max of x over lanes col, col + 16, col + 32, col + 48 (col = lane % 16).
 __device__ __forceinline__ float max_over_rows(float x) {
@@ -286,9 +297,9 @@ __device__ __forceinline__ constexpr int partial_coord(int at) {
 // One workgroup's share: split `split` of list `a` (a C4 top-k list through
 // the block table, or with a.block_table == nullptr a list of pool slots), for
 // kHG groups of 16 heads: every expanded record serves all of them.
-template <bool kPacked, int kHG, bool kPlanes = false, bool kLong = false, bool kPos = false,
+template <bool kPacked, int kHG, bool kPlanes = false, Len kLen = kShort, bool kPos = false,
           bool kHelp = false>
-__device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>* sm,
+__device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked, kLen>* sm,
                                           const int split) {
   static_assert(!kHelp || kHG == 1, "tail waves: 16-head workgroups");
   static_assert(kPacked || !kPlanes, "planes hold Packed records");
@@ -329,19 +340,21 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
   // arguments alone, so the consumers' Q loads start at once.
   //
   // Packed workgroups with tail waves (eight waves) on splits of several
-  // stages of at most 512 records: the tail waves take hardware waves 4 and 5
+  // stages whose record table is not refilled: the tail waves take hardware waves 4 and 5
   // (beside the consumers on SIMDs 0 and 1) and producers 2 and 3 waves 6 and
   // 7 (two producers on each of SIMDs 2 and 3). A consumer slows less beside
   // a tail wave than beside a producer: B=64 29.7 -> 28.8 us (table) and 28.4
-  // -> 28.0 us (positions). Long splits (B=128 x next-n 2 94 -> 98-102 us)
-  // and single-stage splits (B=1) keep the default placement.
+  // -> 28.0 us (positions). Refilled splits, whose first consumer has the
+  // refill to do as well (B=128 x next-n 2, when it was refilled, 94 -> 98-102
+  // us), and single-stage splits (B=1) keep the default placement.
   const int wv_hw = uniform(tid >> 6);
   const bool several = ((int)a.topk + kPcStage - 1) / kPcStage > a.splits;
   const bool remap = !kPacked && kHG == 1 && several;
-  const bool tail_remap = kHelp && kPacked && !kLong && several;
+  const bool tail_remap = kHelp && kPacked && kLen != kRefill && several;
   const int wv = remap ? (wv_hw == 2 ? 0 : wv_hw == 3 ? 1 : wv_hw < 2 ? wv_hw + 2 : wv_hw)
                  : tail_remap && wv_hw >= 4 ? (wv_hw ^ 2)
                                             : wv_hw;
+  constexpr int kTab = PcShared<kPacked, kLen>::kTab;
   const int64_t t = blockIdx.y;
   const int splits = a.splits, topk = (int)a.topk;
   const int64_t head_wg = (int64_t)blockIdx.z * 16 * kHG;
@@ -360,6 +373,8 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
 
   // ---- setup: record metadata, selectors ----
   const uint64_t stand_in = (uint64_t)a.q | 1u;
+  // table mode: RoPE row of record slot i (256 bytes; a table is present)
+  auto rope_row = [&](int i) { return (uint64_t)a.freqs + ((uint64_t)aux_tab[i] << 10); };
   const bool paged = a.block_table != nullptr;
   // table entry of record slot i from its top-k entry r (< 0: none) and, for
   // a paged pool, its block-table entry pv (meaningful only when in_table(r))
@@ -379,7 +394,7 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
     // rows sit at a quarter and a 32nd of the values offset in their planes
     const uint8_t* pg = kPlanes ? a.pool + (ok ? page : 0) * 64 * kCodeBytes
                                 : a.pool + (ok ? page : 0) * G::kPage;
-    const int slot = i & (kPcMaxChunk - 1);
+    const int slot = i & (kTab - 1);
     row_tab[slot] = ok ? (uint64_t)(pg + (r & 63) * (kPlanes ? kCodeBytes : G::kData)) |
                              (kPacked ? 0 : (uint64_t)(r & 63) << 58)
                        : stand_in;
@@ -387,7 +402,7 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
     // record, Q without a table); position mode: the position 4 r as a float
     // (0 for an invalid record, whose tail is zero)
     if (kPacked && kPos) aux_tab[slot] = f2u(ok ? (float)(4 * r) : 0.0f);
-    else if (kPacked) aux_tab[slot] = a.freqs ? (uint64_t)(a.freqs + (ok ? r : 0) * 4 * 64) : (uint64_t)a.q;
+    else if (kPacked) aux_tab[slot] = ok ? (uint32_t)r : 0u;
   };
   // The first kPcMaxChunk slots, by all waves but the consumers. The list's
   // length, its top-k entries and, for tables of at most kBtCache columns, the
@@ -398,7 +413,7 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
   // instead of four (length, sequence length, top-k entries, block table).
   // Wider tables look their entries up in memory, one round trip more.
   constexpr int kBuilders = kPcThreads - 64 * kPcConsumers;
-  constexpr int kEntries = (kPcMaxChunk + kBuilders - 1) / kBuilders;  // per thread
+  constexpr int kEntries = (kTab + kBuilders - 1) / kBuilders;  // per thread
   constexpr int kBtLoads = (kBtCache + kBuilders - 1) / kBuilders;
   const int btid = (wv - kPcConsumers) * 64 + lane;
   const bool builder = wv >= kPcConsumers;
@@ -471,7 +486,7 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
 #pragma unroll
     for (int j = 0; j < kEntries; ++j) {
       const int i = btid + j * kBuilders;
-      if (i < kPcMaxChunk) put_entry(i, list_pos(i) < len ? r0[j] : -1, pv[j], in_table);
+      if (i < kTab) put_entry(i, list_pos(i) < len ? r0[j] : -1, pv[j], in_table);
     }
   };
   auto build_table = [&]() {
@@ -503,17 +518,17 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
   block_sync_lds();
   if constexpr (kPos) asm volatile("" : "+v"(theta), "+v"(theta2));
 
-  // Splits of more than kPcMaxChunk records: consumer 0 refills the table
+  // Refilled splits (kRefill, of more records than the table): consumer 0 refills the table
   // ring ahead of the producers, after its MFMA work of each step s. It
   // copies the top-k entries of stage s + 6 into LDS, copies the block-table
   // entries of stage s + 5 (from the top-k entries copied a step earlier), and
   // writes the table entries of stage s + 4, whose copies the producers issue
-  // at step s + 1, after the barrier. Slot i % kPcMaxChunk then belongs to
+  // at step s + 1, after the barrier. Slot i % kTab then belongs to
   // stage i / kPcStage - 16, consumed at step s - 11. The copies go through
   // inline assembly with this wave's own waits, so the compiler adds none
   // before the MFMA loop's transposed LDS reads.
-  constexpr int kRingStages = kPcMaxChunk / kPcStage;
-  const bool long_split = kLong && stages > kRingStages;
+  constexpr int kRingStages = kTab / kPcStage;
+  const bool long_split = kLen == kRefill && stages > kRingStages;
   auto refill = [&](int s) {
     wait_vm();  // this wave's copies of the previous step have landed
     const int ln = opaque_lane();
@@ -600,8 +615,8 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
       // LDS copies, so the compiler's own waits for these loads are exact.
       using Rows = f32x4[4];
       auto tload = [&](int s, Rows& r) {
-        const int slot = (s * kPcStage + 8 * pp + pi) & (kPcMaxChunk - 1);
-        const uint64_t row = s < stages ? aux_tab[slot] : (uint64_t)a.q;
+        const int slot = (s * kPcStage + 8 * pp + pi) & (kTab - 1);
+        const uint64_t row = s < stages ? rope_row(slot) : (uint64_t)a.q;
 #pragma unroll
         for (int u = 0; u < 4; ++u)  // global (not flat) loads: counted by vmcnt alone
           r[u] = *(const __attribute__((address_space(1))) f32x4*)(row + 64 * q + 16 * u);
@@ -609,7 +624,7 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
       auto tail = [&](int s, auto bufc, const Rows& rr) {
         constexpr int B = decltype(bufc)::value;
         const uint8_t* st = &raw[pp][B][0] + pi * G::kPitch;
-        const int slot = (s * kPcStage + 8 * pp + pi) & (kPcMaxChunk - 1);
+        const int slot = (s * kPcStage + 8 * pp + pi) & (kTab - 1);
         const uint64_t row = row_tab[slot];
         const bool valid = !(row & 1u), odd = !kPlanes && (row & 8u) != 0;
         const bool sodd = kPlanes ? (((row - (uint64_t)a.pool) >> 8) & 1u) != 0 : odd;
@@ -641,7 +656,7 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
         // without a table)
         float cs[16];
         if constexpr (kPos) {
-          const float pos = u2f((uint32_t)aux_tab[slot]);
+          const float pos = u2f(aux_tab[slot]);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             rope_sincos(pos * theta[e], cs[2 * e + 1], cs[2 * e]);
@@ -722,10 +737,10 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
     // the older consumer waves, while the producers' expansion sets the stage
     // time (interleaved runs: Packed B=64 33.2-33.8 -> 31.3-32.2 us, the
     // reference H64/H128 shapes 0.2-1.5 us faster, Native and B=1 unchanged).
-    // Long splits keep equal priorities: their consumer wave 0 also refills
-    // the record table, and with the producers ahead B=128 x next-n 2 ran 8 %
-    // slower.
-    if constexpr (!kLong) __builtin_amdgcn_s_setprio(2);
+    // Refilled splits keep equal priorities: their consumer wave 0 also refills
+    // the record table, and with the producers ahead B=128 x next-n 2 (then
+    // refilled) ran 8 % slower.
+    if constexpr (kLen != kRefill) __builtin_amdgcn_s_setprio(2);
     const uint8_t* const dummy = (const uint8_t*)a.q;
     // Copies of stage s into ring buffer B: the record table entries first,
     // then a fixed number of copies per stage. Invalid records and slots past
@@ -739,11 +754,11 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
       for (int j = 0; j < G::kCopies; ++j) {
         const int c = lane + 64 * j;
         const int r = c < G::kRecPieces ? c / G::kPieces : 0;
-        const int idx = (rec0 + r) & (kPcMaxChunk - 1);
+        const int idx = (rec0 + r) & (kTab - 1);
         rw[j] = c >= G::kPieceCount ? (uint64_t)a.q : row_tab[idx];
       }
       uint64_t srow = 0;
-      if (!kPacked) srow = row_tab[(rec0 + ((lane >> 1) & 7)) & (kPcMaxChunk - 1)];
+      if (!kPacked) srow = row_tab[(rec0 + ((lane >> 1) & 7)) & (kTab - 1)];
 #pragma unroll
       for (int j = 0; j < G::kCopies; ++j) {
         const int c = lane + 64 * j;
@@ -790,7 +805,7 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
     auto head = [&](int s, auto bufc, Head& h) {
       constexpr int B = decltype(bufc)::value;
       const uint8_t* st = &raw[p][B][0] + pi * G::kPitch;
-      h.row = row_tab[(s * kPcStage + 8 * p + pi) & (kPcMaxChunk - 1)];
+      h.row = row_tab[(s * kPcStage + 8 * p + pi) & (kTab - 1)];
       // a record staged from an odd pool row starts 8 bytes in
 #pragma unroll
       for (int e = 0; e < 4; ++e) h.w[e] = *(const uint32_t*)(st + kCodeBytes + 8 * pw + 4 * e);
@@ -862,7 +877,7 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
     auto rope_slot = [&](int S) { return &sm->rope_ring[(p * 2 + S) * 2 * 1024 + 16 * lane]; };
     auto issue_rope = [&](int s, auto slotc) {
       constexpr int S = decltype(slotc)::value;
-      const uint64_t entry = aux_tab[(s * kPcStage + 8 * p + pi) & (kPcMaxChunk - 1)];
+      const uint64_t entry = rope_row((s * kPcStage + 8 * p + pi) & (kTab - 1));
       const uint64_t row = s < stages ? entry : (uint64_t)a.q;
       const uint32_t base = lds_addr(&sm->rope_ring[(p * 2 + S) * 2 * 1024]);
       dma16((const void*)(row + 32 * pw), base);
@@ -886,7 +901,7 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
       const u32x4 v = *(const u32x4*)tail;
       float cs[8];
       if constexpr (kPos) {  // angle RN(4 r * theta_j) of pairs 4 pw .. 4 pw + 3
-        const float pos = u2f((uint32_t)aux_tab[(s * kPcStage + 8 * p + pi) & (kPcMaxChunk - 1)]);
+        const float pos = u2f(aux_tab[(s * kPcStage + 8 * p + pi) & (kTab - 1)]);
 #pragma unroll
         for (int e = 0; e < 4; ++e) rope_sincos(pos * theta[e], cs[2 * e + 1], cs[2 * e]);
       } else {
@@ -919,7 +934,7 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
         // lane (record i, word w) converts the 64 coordinates of word w; piece
         // pairs in the order (c + w / 2) % 4 keep a record's lanes on distinct banks
         const int ni = lane >> 3, nw = lane & 7;
-        const bool nvalid = !(row_tab[(s * kPcStage + 8 * p + ni) & (kPcMaxChunk - 1)] & 1u);
+        const bool nvalid = !(row_tab[(s * kPcStage + 8 * p + ni) & (kTab - 1)] & 1u);
         const uint8_t* const rb = &raw[p][B][0];
         const uint8_t* nst = rb + ni * G::kPitch;
         uint16_t* const nrow =
@@ -1045,8 +1060,8 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
   auto consume = [&](int sa, int sb, int tile0) {
     const uint16_t* kta = &ktile[sa][0];
     const uint16_t* ktb = &ktile[sb][0];
-    const uint64_t ra = row_tab[(tile0 + col) & (kPcMaxChunk - 1)];
-    const uint64_t rb = row_tab[(tile0 + kT + col) & (kPcMaxChunk - 1)];
+    const uint64_t ra = row_tab[(tile0 + col) & (kTab - 1)];
+    const uint64_t rb = row_tab[(tile0 + kT + col) & (kTab - 1)];
     const uint64_t va = __ballot(lane < kT && !(ra & 1u));
     const uint64_t vb = __ballot(lane < kT && !(rb & 1u));
     const int ko = col * kPcKPitch + kchunk(g);  // chunk 4 ks + g at ko + 16 ks
@@ -1199,79 +1214,79 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked>
       orow[i * kHeadDim + 16 * nt] = __builtin_bit_cast(uint16_t, (__bf16)(o[nt][i] * f[i]));
 }
 
-// kLong: splits may run past kPcMaxChunk records (the table ring refill),
+// kLen: the split length class (refilled splits carry the table refill),
 // compiled apart so that shorter splits carry none of its code. kPos: the
 // RoPE rotation from positions and inverse frequencies instead of table rows.
-template <int kHG, bool kPlanes, bool kLong, bool kPos>
+template <int kHG, bool kPlanes, Len kLen, bool kPos>
 __global__ __launch_bounds__((PcRoles<kHG, kTailWaves<true, kHG>>::kThreads)) void
 packed_decode_pc_kernel(DecodeArgs a) {
-  __shared__ __attribute__((aligned(16))) uint8_t smem[sizeof(PcShared<true>)];
-  decode_pc<true, kHG, kPlanes, kLong, kPos, kTailWaves<true, kHG>>(
-      a, reinterpret_cast<PcShared<true>*>(smem), blockIdx.x);
+  __shared__ __attribute__((aligned(16))) uint8_t smem[sizeof(PcShared<true, kLen>)];
+  decode_pc<true, kHG, kPlanes, kLen, kPos, kTailWaves<true, kHG>>(
+      a, reinterpret_cast<PcShared<true, kLen>*>(smem), blockIdx.x);
 }
-template <int kHG, bool kLong>
+template <int kHG, Len kLen>
 __global__ __launch_bounds__(PcRoles<kHG>::kThreads) void native_decode_pc_kernel(DecodeArgs a) {
-  __shared__ __attribute__((aligned(16))) uint8_t smem[sizeof(PcShared<false>)];
-  decode_pc<false, kHG, false, kLong>(a, reinterpret_cast<PcShared<false>*>(smem), blockIdx.x);
+  __shared__ __attribute__((aligned(16))) uint8_t smem[sizeof(PcShared<false, kLen>)];
+  decode_pc<false, kHG, false, kLen>(a, reinterpret_cast<PcShared<false, kLen>*>(smem), blockIdx.x);
 }
 // C4 list and window rows in one launch: workgroups x < c4.splits take a C4
 // split, the last column the window rows (Native records, one short split).
-template <bool kPacked, int kHG, bool kPlanes, bool kLong, bool kPos, bool kHelp = false>
+template <bool kPacked, int kHG, bool kPlanes, Len kLen, bool kPos, bool kHelp = false>
 __device__ __forceinline__ void decode_joint(const DecodeArgs& c4, const DecodeArgs& swa) {
-  __shared__ __attribute__((aligned(16))) uint8_t smem[kPcSmemBytes];
+  __shared__ __attribute__((aligned(16))) uint8_t smem[kJointSmemBytes<kPacked, kLen>];
   if ((int)blockIdx.x < c4.splits)
-    decode_pc<kPacked, kHG, kPlanes, kLong, kPos, kHelp>(
-        c4, reinterpret_cast<PcShared<kPacked>*>(smem), blockIdx.x);
+    decode_pc<kPacked, kHG, kPlanes, kLen, kPos, kHelp>(
+        c4, reinterpret_cast<PcShared<kPacked, kLen>*>(smem), blockIdx.x);
   else
-    decode_pc<false, kHG, false, false, false, kHelp>(swa, reinterpret_cast<PcShared<false>*>(smem),
+    decode_pc<false, kHG, false, kShort, false, kHelp>(swa, reinterpret_cast<PcShared<false>*>(smem),
                                                       0);
 }
-template <int kHG, bool kPlanes, bool kLong, bool kPos>
+template <int kHG, bool kPlanes, Len kLen, bool kPos>
 __global__ __launch_bounds__((PcRoles<kHG, kTailWaves<true, kHG>>::kThreads)) void
 packed_swa_decode_pc_kernel(DecodeArgs c4, DecodeArgs swa) {
-  decode_joint<true, kHG, kPlanes, kLong, kPos, kTailWaves<true, kHG>>(c4, swa);
+  decode_joint<true, kHG, kPlanes, kLen, kPos, kTailWaves<true, kHG>>(c4, swa);
 }
-template <int kHG, bool kLong>
+template <int kHG, Len kLen>
 __global__ __launch_bounds__(PcRoles<kHG>::kThreads) void native_swa_decode_pc_kernel(
     DecodeArgs c4, DecodeArgs swa) {
-  decode_joint<false, kHG, false, kLong, false>(c4, swa);
+  decode_joint<false, kHG, false, kLen, false>(c4, swa);
 }
 
 // The workgroup kernel for a format, storage layout, head grouping, split
 // length and (Packed) RoPE source.
 using SplitKernel = void (*)(DecodeArgs);
 using JointKernel = void (*)(DecodeArgs, DecodeArgs);
-template <bool kLong, bool kPos>
+template <Len kLen, bool kPos>
 SplitKernel packed_split_kernel(bool planes, int hg) {
   if (planes)
-    return hg == 2 ? packed_decode_pc_kernel<2, true, kLong, kPos>
-                   : packed_decode_pc_kernel<1, true, kLong, kPos>;
-  return hg == 2 ? packed_decode_pc_kernel<2, false, kLong, kPos>
-                 : packed_decode_pc_kernel<1, false, kLong, kPos>;
+    return hg == 2 ? packed_decode_pc_kernel<2, true, kLen, kPos>
+                   : packed_decode_pc_kernel<1, true, kLen, kPos>;
+  return hg == 2 ? packed_decode_pc_kernel<2, false, kLen, kPos>
+                 : packed_decode_pc_kernel<1, false, kLen, kPos>;
 }
-template <bool kPacked, bool kLong>
+template <bool kPacked, Len kLen>
 SplitKernel split_kernel(bool planes, int hg, bool pos) {
   if constexpr (!kPacked)
-    return hg == 2 ? native_decode_pc_kernel<2, kLong> : native_decode_pc_kernel<1, kLong>;
+    return hg == 2 ? native_decode_pc_kernel<2, kLen> : native_decode_pc_kernel<1, kLen>;
   else
-    return pos ? packed_split_kernel<kLong, true>(planes, hg)
-               : packed_split_kernel<kLong, false>(planes, hg);
+    return pos ? packed_split_kernel<kLen, true>(planes, hg)
+               : packed_split_kernel<kLen, false>(planes, hg);
 }
-template <bool kLong, bool kPos>
+template <Len kLen, bool kPos>
 JointKernel packed_joint_kernel(bool planes, int hg) {
   if (planes)
-    return hg == 2 ? packed_swa_decode_pc_kernel<2, true, kLong, kPos>
-                   : packed_swa_decode_pc_kernel<1, true, kLong, kPos>;
-  return hg == 2 ? packed_swa_decode_pc_kernel<2, false, kLong, kPos>
-                 : packed_swa_decode_pc_kernel<1, false, kLong, kPos>;
+    return hg == 2 ? packed_swa_decode_pc_kernel<2, true, kLen, kPos>
+                   : packed_swa_decode_pc_kernel<1, true, kLen, kPos>;
+  return hg == 2 ? packed_swa_decode_pc_kernel<2, false, kLen, kPos>
+                 : packed_swa_decode_pc_kernel<1, false, kLen, kPos>;
 }
-template <bool kPacked, bool kLong>
+template <bool kPacked, Len kLen>
 JointKernel joint_kernel(bool planes, int hg, bool pos) {
   if constexpr (!kPacked)
-    return hg == 2 ? native_swa_decode_pc_kernel<2, kLong> : native_swa_decode_pc_kernel<1, kLong>;
+    return hg == 2 ? native_swa_decode_pc_kernel<2, kLen> : native_swa_decode_pc_kernel<1, kLen>;
   else
-    return pos ? packed_joint_kernel<kLong, true>(planes, hg)
-               : packed_joint_kernel<kLong, false>(planes, hg);
+    return pos ? packed_joint_kernel<kLen, true>(planes, hg)
+               : packed_joint_kernel<kLen, false>(planes, hg);
 }
 
 // Butterfly over the wave's 64 lanes with the pairing of xor distances 1, 2,
@@ -1438,7 +1453,7 @@ struct Plan {
 // Split plan: about one workgroup per CU (256 CUs), whole 32-record stages per
 // split and at most max_splits splits (the combine merges at most kMaxSplits
 // partial slots per row, the window rows' slot included). A split may hold
-// more than kPcMaxChunk records (its table ring is refilled as it goes), so
+// more than kPcMaxChunk records (Len), so
 // a batch that fills the round on its own takes one split per token: one
 // round of workgroups and no partials to merge.
 // 16-head groups per workgroup. Two groups share every expanded record (half
@@ -1588,7 +1603,9 @@ int launch_decode(const uint16_t* q, int64_t batch, int64_t q_len, int64_t heads
                    : kPacked ? PcRoles<1, true>::kThreads
                              : PcRoles<1>::kThreads);
   const unsigned zblocks = (unsigned)(heads / (16 * hg));
-  const bool lng = plan.chunk > kPcMaxChunk;
+  const Len len = plan.chunk <= kPcMaxChunk             ? kShort
+                  : kPacked && plan.chunk <= table_slots(kWhole) ? kWhole
+                                                      : kRefill;
   if (w.topk > 0) {
     // the window rows are one more split, read by the Native path of the same launch
     DecodeArgs b = a;
@@ -1610,13 +1627,15 @@ int launch_decode(const uint16_t* q, int64_t batch, int64_t q_len, int64_t heads
     b.splits_magic = 65536;
     b.ws_base = plan.splits;
     const dim3 grid((unsigned)slots, (unsigned)tokens, zblocks);
-    const JointKernel kern = lng ? joint_kernel<kPacked, true>(src.planes(), hg, pos)
-                                 : joint_kernel<kPacked, false>(src.planes(), hg, pos);
+    const JointKernel kern = len == kShort   ? joint_kernel<kPacked, kShort>(src.planes(), hg, pos)
+                             : len == kWhole ? joint_kernel<kPacked, kPacked ? kWhole : kRefill>(src.planes(), hg, pos)
+                                             : joint_kernel<kPacked, kRefill>(src.planes(), hg, pos);
     hipLaunchKernelGGL(kern, grid, block, 0, s, a, b);
   } else {
     const dim3 grid((unsigned)plan.splits, (unsigned)tokens, zblocks);
-    const SplitKernel kern = lng ? split_kernel<kPacked, true>(src.planes(), hg, pos)
-                                 : split_kernel<kPacked, false>(src.planes(), hg, pos);
+    const SplitKernel kern = len == kShort   ? split_kernel<kPacked, kShort>(src.planes(), hg, pos)
+                             : len == kWhole ? split_kernel<kPacked, kPacked ? kWhole : kRefill>(src.planes(), hg, pos)
+                                             : split_kernel<kPacked, kRefill>(src.planes(), hg, pos);
     hipLaunchKernelGGL(kern, grid, block, 0, s, a);
   }
   if (hipGetLastError() != hipSuccess) return RM_ERR_LAUNCH;

@@ -530,3 +530,26 @@ def test_decode_combine_split_counts(tokens, topk):
     out, lse = run_decode(c)
     ref, ref_lse = oracle_decode(c)
     per_row_check(out, ref, lse, ref_lse)
+
+
+# ---- whole and refilled tables around 512 and 2,048 records a split -----------------------
+
+@pytest.mark.parametrize("rope", ["table", "positions"])
+@pytest.mark.parametrize("topk", [513, 2048, 2049, 2400])
+def test_decode_long_split_table_sizes(topk, rope):
+    """One split per token (32 requests x 2 query tokens x 128 heads, 32-head
+    workgroups): tables built whole up to 2,048 records,
+    refilled beyond, and a second pass (q scaled so that later stages exceed
+    the first one's maximum by more than the slack)."""
+    banner(f"decode long-split tables topk={topk} {rope}")
+    ctx = syn.log_uniform_contexts(32, 2500, 3000, 503)
+    c = build_decode_case(ctx, q_len=2, heads=128, topk=topk, seed=503, packed=True)
+    assert remnant.get_decode_metadata(64, 128, topk)[0] == 1
+    c["rope"] = rope
+    lens = c["lens"].reshape(-1)
+    lens[:] = np.minimum(lens, 40)  # most lists short (the oracle's time)
+    lens[[0, 1, 2, 3, 40, 63]] = [topk, 512, 513, 0, topk - 1, topk]
+    c["q"] = (c["q"].float() * 300).to(torch.bfloat16)
+    out, lse = run_decode(c)
+    ref, ref_lse = oracle_decode(c)
+    per_row_check(out, ref, lse, ref_lse)
