@@ -844,3 +844,37 @@ def test_bulk_workload_1m_records_pack_and_reconstruct_sampled():
                                 np.array([pick.size], np.int32))
     got_rows = syn.bf16_bits(out.index_select(0, pick_d))
     assert np.array_equal(got_rows, rows)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [1, 5, 4097, 131073])
+def test_native_store_sizes_and_non_finite_rows(n, dtype):
+    """One row, one more than a workgroup's four, runs of several rows a wave
+    and the streaming form past 131,072 rows; skipped slots and positions among
+    them. Rows with an infinity or NaN are stored beside the others without
+    disturbing them (their own bytes have no defined value)."""
+    x = syn.latents(n, seed=77).to(dtype)
+    special = np.arange(2, n, 997)
+    for i, v in zip(special, np.resize([np.inf, -np.inf, np.nan], special.size)):
+        x[int(i), int(i) % 512] = float(v)
+    pages = (n + 63) // 64 + 1
+    rng = np.random.default_rng(n)
+    slots = rng.permutation(pages * 64)[:n].astype(np.int32)
+    pos = np.arange(n, dtype=np.int32) % 1000
+    slots[3::31], pos[4::37] = -1, 1000  # skipped
+    freqs = syn.rope_freqs(4000)
+    pool = remnant.LatentPool(pages, fmt="native", device=DEV)
+    remnant.native_store_rows(x.to(DEV), torch.ones(512, device=DEV), 1e-6,
+                              torch.from_numpy(slots).to(DEV), torch.from_numpy(pos).to(DEV),
+                              freqs.to(DEV), pool)
+    ref = np.zeros((pages, 37376), np.uint8)
+    oracle.native_pack_rows_paged(x.float().numpy(), np.ones(512, np.float32), 1e-6, slots, pos,
+                              torch.view_as_real(freqs).numpy(), ref)
+    got = pool.layer().cpu().numpy().copy()
+    for i in special:  # not compared
+        s = int(slots[i])
+        if s >= 0:
+            for a in (got, ref):
+                a[s // 64, s % 64 * 576:s % 64 * 576 + 576] = 0
+                a[s // 64, 36864 + s % 64 * 8:36864 + s % 64 * 8 + 8] = 0
+    assert np.array_equal(got, ref)
