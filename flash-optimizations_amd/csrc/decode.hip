@@ -418,7 +418,8 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked,
   const int btid = (wv - kPcConsumers) * 64 + lane;
   const bool builder = wv >= kPcConsumers;
   const int32_t* const none = (const int32_t*)a.q;
-  const bool bt_cached = paged && a.max_blocks <= kBtCache;
+  // (a table of no columns, or of a call without lists, has no row to load)
+  const bool bt_cached = paged && topk > 0 && a.max_blocks > 0 && a.max_blocks <= kBtCache;
   int32_t* const bt_lds = (int32_t*)&ktile[0][0];
   static_assert(sizeof(ktile) >= kBtLoads * kBuilders * sizeof(int32_t), "row in the K ring");
   // (scalar loads)
@@ -432,7 +433,7 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked,
 #pragma unroll
     for (int j = 0; j < kEntries; ++j) r0[j] = list[min((uint32_t)list_pos(btid + j * kBuilders), last)];
     const int32_t* const row = bt_cached ? a.block_table + b * a.bt_stride : none;
-    const uint32_t last_col = bt_cached && a.max_blocks > 0 ? (uint32_t)a.max_blocks - 1 : 0;
+    const uint32_t last_col = bt_cached ? (uint32_t)a.max_blocks - 1 : 0;
 #pragma unroll
     for (int j = 0; j < kBtLoads; ++j) bv[j] = row[min((uint32_t)(btid + j * kBuilders), last_col)];
   };

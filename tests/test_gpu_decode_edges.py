@@ -26,6 +26,7 @@ import torch
 
 import oracle
 import remnant
+from remnant import _lib
 from remnant import synthetic as syn
 from test_gpu_parity import (COS_MIN, DEV, OUT_TOL, W1, assert_pool_equal, build_decode_case,
                              check_decode, gpu_pack, oracle_decode, oracle_pack, run_decode)
@@ -553,3 +554,35 @@ def test_decode_long_split_table_sizes(topk, rope):
     out, lse = run_decode(c)
     ref, ref_lse = oracle_decode(c)
     per_row_check(out, ref, lse, ref_lse)
+
+
+# ---- block table without columns -------------------------------------------------------------
+
+@pytest.mark.parametrize("packed", [True, False], ids=["direct", "native"])
+def test_decode_block_table_without_columns(packed):
+    """A block table of no columns (max_blocks 0, any stride; through the C ABI,
+    since an empty torch tensor has no address) maps no record and none of it is
+    read: every list comes out empty, output zero and LSE the sink's."""
+    banner(f"decode block table without columns packed={packed}")
+    batch, heads, topk = 3, 16, 64
+    lib = _lib.load()
+    pool = remnant.LatentPool(2, fmt="remnant" if packed else "native", device=DEV)
+    q = torch.randn(batch, heads, 512, device=DEV).to(torch.bfloat16)
+    idx = torch.arange(topk, dtype=torch.int32, device=DEV).repeat(batch, 1).contiguous()
+    sink = torch.randn(heads, device=DEV)
+    table = torch.zeros(4, dtype=torch.int32, device=DEV)  # an address; column 0 would be page 0
+    need = remnant.get_decode_metadata(batch, heads, topk)[1]
+    ws = torch.empty(max(need, 1), dtype=torch.uint8, device=DEV)
+    for stride in (0, 1):
+        out = torch.full((batch, heads, 512), 7.0, dtype=torch.bfloat16, device=DEV)
+        lse = torch.zeros(batch, heads, device=DEV)
+        args = [q.data_ptr(), batch, 1, heads, pool.buffer.data_ptr(), 2, table.data_ptr(), stride, 0,
+                None, idx.data_ptr(), topk, None, sink.data_ptr()]
+        rope = [None, 0, None] if packed else []
+        fn = lib.rm_remnant_sparse_decode_fwd if packed else lib.rm_native_sparse_decode_fwd
+        assert fn(*args, *rope, 0.1, out.data_ptr(), lse.data_ptr(), ws.data_ptr(), need,
+                  torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        assert not out.any()
+        # lse = ln(exp(sink)) through base 2: a few FP32 roundings of |sink| < 8
+        assert (lse - sink).abs().max() <= 8 * 2.0 ** -22
