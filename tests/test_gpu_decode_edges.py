@@ -586,3 +586,29 @@ def test_decode_block_table_without_columns(packed):
         assert not out.any()
         # lse = ln(exp(sink)) through base 2: a few FP32 roundings of |sink| < 8
         assert (lse - sink).abs().max() <= 8 * 2.0 ** -22
+
+
+# ---- short lists in whole tables ----------------------------------------------------------------
+
+@pytest.mark.parametrize("rope", ["table", "positions"])
+@pytest.mark.parametrize("heads", [16, 64])
+def test_decode_short_lists_in_whole_tables(heads, rope):
+    """One split per token at top-k 2048 (256 tokens x 16 heads, 128 x 64 heads in
+    32-head workgroups), lists on both sides of each stage and of where the
+    set-up writes two slots a thread or all of them (12 stages at 32 heads, 20
+    at 16), after lists that filled the table's LDS."""
+    banner(f"decode short lists in whole tables heads={heads} {rope}")
+    batch, q_len = (128, 2) if heads == 16 else (64, 2)
+    topk = 2048
+    ctx = syn.log_uniform_contexts(batch, 2100, 2500, 521)
+    c = build_decode_case(ctx, q_len=q_len, heads=heads, topk=topk, seed=521, packed=True)
+    assert remnant.get_decode_metadata(batch * q_len, heads, topk)[0] == 1
+    c["rope"] = rope
+    run_decode(c)  # full lists
+    lens = c["lens"].reshape(-1)
+    edges = [0, 1, 31, 32, 33, 352, 353, 383, 384, 385, 416, 417, 511, 512, 513, 608, 609, 639, 640,
+             641, 672, 673]
+    lens[:] = np.resize(edges, lens.size)
+    out, lse = run_decode(c)
+    ref, ref_lse = oracle_decode(c)
+    per_row_check(out, ref, lse, ref_lse)
