@@ -97,7 +97,7 @@ struct DecodeArgs {
   float scale_log2;
   uint64_t q_len_magic;  // ceil(2^32 / q_len): token t < 2^16 is of request t * q_len_magic >> 32
   int64_t heads;
-  int chunk;       // records per split (multiple of 32)
+  int chunk;       // records per split of a full list (multiple of 32)
   int splits;      // splits of this list (workgroups along x)
   uint32_t splits_magic;  // ceil(2^16 / splits): x / splits = x * splits_magic >> 16 for x < 2^10
   int ws_splits;   // partial slots per row in the workspace; 0: finalise in place
@@ -325,7 +325,7 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked,
   asm volatile("" ::"s"(a.q), "s"(a.pool), "s"(a.pool_pages), "s"(a.pool_rows), "s"(a.block_table),
                "s"(a.bt_stride), "s"(a.max_blocks), "s"(a.seqlens), "s"(a.indices), "s"(a.topk),
                "s"(a.topk_length), "s"(a.freqs), "s"(a.freq_rows), "s"(a.inv_freq),
-               "s"(a.q_len_magic), "s"(a.heads), "s"(a.splits), "s"(a.splits_magic));
+               "s"(a.q_len_magic), "s"(a.heads), "s"(a.chunk), "s"(a.splits), "s"(a.splits_magic));
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   // Role index of this wave. A workgroup's waves fill SIMDs 0..3 in order
@@ -354,22 +354,28 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked,
   const int wv = remap ? (wv_hw == 2 ? 0 : wv_hw == 3 ? 1 : wv_hw < 2 ? wv_hw + 2 : wv_hw)
                  : tail_remap && wv_hw >= 4 ? (wv_hw ^ 2)
                                             : wv_hw;
-  constexpr int kTab = PcShared<kPacked, kLen>::kTab;
   const int64_t t = blockIdx.y;
-  const int splits = a.splits, topk = (int)a.topk;
+  const int topk = (int)a.topk;
   const int64_t head_wg = (int64_t)blockIdx.z * 16 * kHG;
   // a consumer's 16 heads (consumers 2 hg and 2 hg + 1 serve group hg)
   const int64_t head0 = head_wg + (wv < kPcConsumers ? 16 * (wv >> 1) : 0);
   const int64_t b = (int64_t)(((uint64_t)t * a.q_len_magic) >> 32);
 
-  // Stage j of this split is stage j * splits + split of the list: where a
-  // record sits does not depend on the list's valid length, so the top-k
-  // entries are requested together with the length, and a short list still
-  // spreads evenly over the splits (to within one stage).
-  auto list_pos = [&](int i) {
-    return ((i >> 5) * splits + split) * kPcStage + (i & (kPcStage - 1));
-  };
-  static_assert(kPcStage == 32, "list_pos");
+  // The table is built from kTab list entries loaded together with the list's
+  // length, from list position w0 on. With n valid entries the split takes its
+  // share [k0, k0 + n) of the list (below), k0 <= split * a.chunk and k0 + n <=
+  // (split + 1) * a.chunk whatever the length: w0 puts the window's end there,
+  // so that it holds the share of most shorter lists too (of every list of at
+  // most kTab entries). Otherwise the entries are loaded again from k0, one
+  // memory round trip more. (Dealing the stages out in turn, stage j of a split
+  // being stage j * splits + split of the list, needs no second load either way,
+  // but a split then takes its softmax reference from other records and outputs
+  // differ in their last bits. Full lists take the same time; 317 of 512 records
+  // at 64 heads x B=16, whose three splits then hold 4, 3 and 3 stages instead
+  // of 4, 4 and 2, 64.2 us dealt out and 65.0 us like this, four layers.)
+  constexpr int kTab = PcShared<kPacked, kLen>::kTab;
+  const int k0_full = split * a.chunk;
+  int w0 = max(0, k0_full - max(0, kTab - a.chunk));
 
   // ---- setup: record metadata, selectors ----
   const uint64_t stand_in = (uint64_t)a.q | 1u;
@@ -405,8 +411,9 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked,
     else if (kPacked) aux_tab[slot] = ok ? (uint32_t)r : 0u;
   };
   // The table's slots (the first ones of a refilled split), by all waves but
-  // the consumers. The list's length, its top-k entries and, for tables of at most kBtCache columns, the
-  // request's block-table row are requested side by side, every load
+  // the consumers. The list's length, its top-k entries and, for tables of at
+  // most kBtCache columns, the request's block-table row are requested side by
+  // side, every load
   // unconditional (clamped to what is there) so that no wait comes between
   // two; the row is then looked up in LDS (in the K ring, idle here). The
   // records' addresses are one memory round trip away from the arguments
@@ -427,11 +434,14 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked,
   const int len_raw = *(const_i32*)(uintptr_t)(a.topk_length ? a.topk_length + t : none);
   const int seq_raw = *(const_i32*)(uintptr_t)(a.seqlens ? a.seqlens + b : none);
   int32_t r0[kEntries], bv[kBtLoads];
-  auto load_entries = [&]() {
+  auto load_list = [&]() {
     const int32_t* const list = topk > 0 ? a.indices + t * topk : none;
     const uint32_t last = topk > 0 ? topk - 1 : 0;
 #pragma unroll
-    for (int j = 0; j < kEntries; ++j) r0[j] = list[min((uint32_t)list_pos(btid + j * kBuilders), last)];
+    for (int j = 0; j < kEntries; ++j) r0[j] = list[min((uint32_t)(w0 + btid + j * kBuilders), last)];
+  };
+  auto load_entries = [&]() {
+    load_list();
     const int32_t* const row = bt_cached ? a.block_table + b * a.bt_stride : none;
     const uint32_t last_col = bt_cached ? (uint32_t)a.max_blocks - 1 : 0;
 #pragma unroll
@@ -459,12 +469,16 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked,
     }
     sel_tab[e] = sel;
   }
-  // valid entries of this token's list, and this split's stages of them
+  // this token's valid entries in whole stages, spread evenly over the splits
+  // (at most a.chunk each, since len <= topk): a short list finishes early in
+  // every split instead of emptying the last ones
   const int len = !a.topk_length || len_raw > topk ? topk : max(len_raw, 0);
   const int len_stages = (len + kPcStage - 1) / kPcStage;
-  const int stages = len_stages > split
-                         ? (int)(((uint32_t)(len_stages - 1 - split) * a.splits_magic) >> 16) + 1
-                         : 0;
+  const int chunk =
+      len > 0 ? ((int)(((uint32_t)(len_stages - 1) * a.splits_magic) >> 16) + 1) * kPcStage : 0;
+  const int k0 = split * chunk;
+  const int n = max(0, min(chunk, len - k0));
+  const int stages = (n + kPcStage - 1) / kPcStage;
   const int64_t seqlen = a.seqlens ? seq_raw : INT64_MAX;
   // whether logical record r of request b has a block-table entry to read
   auto in_table = [&](int64_t r) { return r >= 0 && r < seqlen && (r >> 6) < a.max_blocks; };
@@ -480,11 +494,15 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked,
         pv[j] = *(paged && in_table(r0[j]) ? a.block_table + (b * a.bt_stride + (r0[j] >> 6)) : none);
 #pragma unroll
     for (int j = 0; j < kCount; ++j) {
-      const int i = btid + j * kBuilders;
-      if (i < kTab) put_entry(i, list_pos(i) < len ? r0[j] : -1, pv[j], in_table);
+      const int i = w0 - k0 + btid + j * kBuilders;  // (slot i % kTab: the window holds each once)
+      if (btid + j * kBuilders < kTab) put_entry(i, (uint32_t)i < (uint32_t)n ? r0[j] : -1, pv[j], in_table);
     }
   };
   auto make_entries = [&]() {
+    if (builder && k0 < w0 && n > 0) {  // the share starts before the window
+      w0 = k0;
+      load_list();
+    }
     if (bt_cached) {
       if (builder) {
 #pragma unroll
@@ -501,7 +519,7 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked,
     // slot written, 11.1 with two a thread; 128 x 64 heads 15.0 and 13.3; full
     // lists unchanged).
     if constexpr (kLen == kWhole) {
-      if ((stages + G::kDepth) * kPcStage <= 2 * kBuilders) {
+      if (w0 == k0 && (stages + G::kDepth) * kPcStage <= 2 * kBuilders) {
         put_entries(std::integral_constant<int, 2>{});
         return;
       }
@@ -554,13 +572,13 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked,
     int q = s + 4;
     if (q >= kRingStages && q < stages && ln < kPcStage) {
       const int i = q * kPcStage + ln;
-      const int64_t r = list_pos(i) < len ? (int64_t)sm->idx_ring[q % 3][ln] : -1;
+      const int64_t r = i < n ? (int64_t)sm->idx_ring[q % 3][ln] : -1;
       put_entry(i, r, sm->bt_ring[q % 3][ln], in_table);
     }
     q = s + 5;
     if (q >= kRingStages && q < stages) {
       const int i = q * kPcStage + ln;
-      const int64_t r = ln < kPcStage && list_pos(i) < len ? (int64_t)sm->idx_ring[q % 3][ln] : -1;
+      const int64_t r = ln < kPcStage && i < n ? (int64_t)sm->idx_ring[q % 3][ln] : -1;
       const int32_t* src = paged && in_table(r) ? a.block_table + (b * a.bt_stride + (r >> 6))
                                                 : (const int32_t*)a.q;
       dma4_opaque(src, lds_addr(&sm->bt_ring[q % 3][0]));
@@ -568,8 +586,8 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked,
     q = s + 6;
     if (q >= kRingStages && q < stages) {
       const int i = q * kPcStage + ln;
-      const int32_t* src = ln < kPcStage && list_pos(i) < len ? a.indices + (t * a.topk + list_pos(i))
-                                                              : (const int32_t*)a.q;
+      const int32_t* src = ln < kPcStage && i < n ? a.indices + (t * a.topk + k0 + i)
+                                                  : (const int32_t*)a.q;
       dma4_opaque(src, lds_addr(&sm->idx_ring[q % 3][0]));
     }
   };

@@ -494,12 +494,12 @@ def test_native_decode_pool_beyond_4gib_offsets():
 # ---- block-table width: rows looked up in LDS up to 1,024 columns -------------------------
 
 @pytest.mark.parametrize("packed", [True, False], ids=["direct", "native"])
-def test_decode_block_table_width_and_interleaved_stages(packed):
+def test_decode_block_table_width(packed):
     """Requests of 1 to 700 records, three query tokens each (a token's request
-    by the q_len reciprocal), list lengths that end in every position of the
-    splits' interleaved stages. The table as it is, padded to 1,024 columns
-    (looked up in LDS) and to 1,025 (looked up in memory): the same bits, and
-    within tolerance of the oracle."""
+    by the q_len reciprocal), 14 splits of one stage each, lists that end at and
+    beside stage ends. The table as it is, padded to 1,024 columns (looked up in
+    LDS) and to 1,025 (looked up in memory): the same bits, and within tolerance
+    of the oracle."""
     banner(f"decode block-table width packed={packed}")
     ctx = [700, 1, 64, 65, 333]
     c = build_decode_case(ctx, q_len=3, heads=16, topk=417, seed=487, packed=packed)
@@ -612,3 +612,72 @@ def test_decode_short_lists_in_whole_tables(heads, rope):
     out, lse = run_decode(c)
     ref, ref_lse = oracle_decode(c)
     per_row_check(out, ref, lse, ref_lse)
+
+
+# ---- the splits' shares of a list ---------------------------------------------------------------
+
+def run_split_lse(c, splits):
+    """Output, LSE and the split partials' LSEs [tokens, splits, heads] (natural
+    log, without the sink) of a decode, from the caller's workspace."""
+    batch, q_len, heads = c["q"].shape[:3]
+    tokens, topk = batch * q_len, c["idx"].shape[-1]
+    got, need = remnant.get_decode_metadata(tokens, heads, topk)
+    assert got == splits
+    ws = torch.zeros(need, dtype=torch.uint8, device=DEV)
+    kw = dict(seqlens=torch.tensor(c["contexts"], dtype=torch.int32, device=DEV),
+              topk_length=torch.from_numpy(c["lens"]).to(DEV), sink=c["sink"].to(DEV),
+              workspace=ws)
+    fn = remnant.native_sparse_decode_fwd
+    if c["packed"]:
+        fn = remnant.remnant_sparse_decode_fwd
+        kw["freqs_cis"] = c["freqs"].to(DEV)
+    out, lse = fn(c["q"].to(DEV), c["pool"], torch.from_numpy(c["table"]).to(DEV),
+                  torch.from_numpy(c["idx"]).to(DEV), **kw)
+    torch.cuda.synchronize()
+    parts = ws.view(torch.float32)[tokens * splits * heads * 512:].cpu().numpy()
+    return (out.float().cpu().numpy(), lse.cpu().numpy(),
+            parts[:tokens * splits * heads].reshape(tokens, splits, heads) * np.log(2.0))
+
+
+@pytest.mark.parametrize("packed", [True, False], ids=["direct", "native"])
+@pytest.mark.parametrize("batch,q_len,heads,topk,splits",
+                         [(5, 3, 16, 417, 14), (8, 2, 64, 317, 4), (32, 2, 16, 2048, 4),
+                          (64, 2, 16, 2048, 2), (64, 2, 16, 4160, 2)],
+                         ids=["one-stage", "317", "512-a-split", "1024-a-split", "2080-a-split"])
+def test_decode_splits_take_consecutive_shares(batch, q_len, heads, topk, splits, packed):
+    """Split s of a list of n records in m = ceil(n / 32) stages attends records
+    [s c, (s + 1) c) of it, c = 32 ceil(m / splits): its partial's LSE is the
+    oracle's over that share alone. Lengths at and beside every stage count at
+    which a share moves, in tables of 512 slots, of 2,048 (Packed, two splits of
+    1,024) and refilled (Native at 1,024 and both formats at 2,080 records a
+    split, two splits)."""
+    banner(f"decode split shares {batch}x{q_len}x{heads} topk={topk} packed={packed}")
+    # contexts beyond the top-k (the lists' lengths are set here)
+    ctx = syn.log_uniform_contexts(batch, 4 * topk + 128, 4 * topk + 800, 541)
+    c = build_decode_case(ctx, q_len=q_len, heads=heads, topk=topk, seed=541, packed=packed)
+    lens = c["lens"].reshape(-1)
+    stages = (topk + 31) // 32
+    edges = [0, 1, topk, topk - 1]
+    for m in range(1, stages + 1):
+        if m % splits in (0, 1) or m in (stages - 1, stages):
+            edges += [32 * m - 1, 32 * m, 32 * m + 1]
+    edges = np.unique(np.minimum(edges, topk))
+    pick = np.linspace(0, edges.size - 1, min(lens.size, edges.size)).astype(int)
+    lens[:] = np.resize(edges[pick], lens.size)
+    out, lse, parts = run_split_lse(c, splits)
+    ref, ref_lse = oracle_decode(c)
+    per_row_check(out, ref, lse, ref_lse)
+    full, sink = c["idx"], c["sink"]
+    share = 32 * (-(-(-(-lens // 32)) // splits))
+    c["sink"] = None
+    for s in range(splits):
+        start = np.minimum(s * share, lens)
+        count = np.minimum(share, lens - start)
+        idx = full.reshape(lens.size, topk)
+        at = np.minimum(start[:, None] + np.arange(max(int(count.max()), 1)), topk - 1)
+        c["idx"] = np.take_along_axis(idx, at, axis=1).reshape(*full.shape[:2], -1).copy()
+        c["lens"] = count.astype(np.int32).reshape(np.shape(c["lens"]))
+        part_lse = oracle_decode(c)[1].reshape(lens.size, heads)
+        empty = count == 0
+        assert np.isneginf(parts[empty, s]).all()
+        assert np.abs(parts[~empty, s] - part_lse[~empty]).max(initial=0) <= OUT_TOL
