@@ -1358,7 +1358,8 @@ __device__ __forceinline__ float lane_of(float x, int l) {
 // kWaveBatch splits are issued together with the split LSEs (lane s holds
 // split s), so a row costs one round trip per kWaveBatch splits.
 // kWaveBatch is 4 for up to four splits and 8 beyond. Loads past the last split
-// repeat it with weight zero: a branch around each would make the kernel, which
+// repeat it and are left out of the sum (not added with weight zero: an infinite
+// partial would become a NaN): a branch around each load would make the kernel, which
 // runs once per row, mostly instruction fetch (with the token and head from the
 // grid instead of a division: decode at B=64 0.55 us less a layer, of 33).
 template <int kWaveBatch>
@@ -1401,7 +1402,8 @@ __global__ __launch_bounds__(256) void combine_wave_kernel(const float* __restri
 #pragma unroll
     for (int u = 0; u < kWaveBatch; ++u) {
       const int sp = s0 + u;
-      const float ww = sp < splits ? lane_of(w, sp) : 0.0f;
+      if (sp >= splits) break;
+      const float ww = lane_of(w, sp);
       a0 += ww * x[2 * u];
       a1 += ww * x[2 * u + 1];
     }
@@ -1430,7 +1432,7 @@ __global__ __launch_bounds__(256) void combine_wave_kernel(const float* __restri
 // partial sums meet in LDS in a fixed order. The split weights come from every
 // split's LSE, read by every wave (lane s holds split s; splits <= 64).
 // kPerWave (4, 8 or 16) is the smallest that covers the splits; loads past the
-// last split repeat it with weight zero, as in combine_wave_kernel.
+// last split repeat it and are left out of the sum, as in combine_wave_kernel.
 constexpr int kCombineSlices = kHeadDim / 64;
 template <int kPerWave>
 __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ ws_o,
@@ -1465,7 +1467,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
 #pragma unroll
   for (int u = 0; u < kPerWave; ++u) {
     const int s = wave + 4 * u;
-    acc += (s < splits ? lane_of(w, s) : 0.0f) * x[u];
+    if (s < splits) acc += lane_of(w, s) * x[u];
   }
   part[wave][lane] = acc;
   __syncthreads();

@@ -681,3 +681,29 @@ def test_decode_splits_take_consecutive_shares(batch, q_len, heads, topk, splits
         empty = count == 0
         assert np.isneginf(parts[empty, s]).all()
         assert np.abs(parts[~empty, s] - part_lse[~empty]).max(initial=0) <= OUT_TOL
+
+
+# ---- combine: an infinite partial ----------------------------------------------------------------
+
+@pytest.mark.parametrize("tokens,topk,splits", [(1, 96, 3), (1, 544, 17), (1, 1056, 33),
+                                                (64, 96, 3), (48, 2048, 6)])
+def test_decode_combine_keeps_infinite_partials(tokens, topk, splits):
+    """Native records whose coordinates are all 448 * 2^119, below the BF16
+    maximum, under q = 0: every weight is 1 and every partial's 448 sums are past
+    the FP32 range. The output is infinite there (not NaN: nothing is added for
+    the loads past the last split), zero in the tail, the LSE ln(topk)."""
+    banner(f"decode combine infinite partials tokens={tokens} topk={topk}")
+    pool = remnant.LatentPool(33, fmt="native", device=DEV)
+    page = torch.zeros(37376, dtype=torch.uint8)
+    page[:36864].view(64, 576)[:, :448] = 0x7E
+    page[36864:].view(64, 8)[:, :7] = 127 + 119
+    pool.buffer[0] = page.to(DEV)
+    q = torch.zeros(tokens, 1, 16, 512, dtype=torch.bfloat16, device=DEV)
+    idx = torch.arange(topk, dtype=torch.int32, device=DEV).repeat(tokens, 1, 1).contiguous()
+    table = torch.arange(33, dtype=torch.int32, device=DEV).repeat(tokens, 1).contiguous()
+    assert remnant.get_decode_metadata(tokens, 16, topk)[0] == splits
+    out, lse = remnant.native_sparse_decode_fwd(q, pool, table, idx)
+    torch.cuda.synchronize()
+    assert (out[..., :448] == float("inf")).all() and not out[..., 448:].any()
+    # log2 of the sum and its conversion to base e: a few FP32 roundings of ln(topk) < 8
+    assert (lse - np.log(topk)).abs().max() <= 8 * 2.0 ** -22
