@@ -570,17 +570,146 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(
   }
 }
 
-// Native records. The next row, its slot and position are in flight while a
-// row is stored (they were loaded one after the other, each a memory round
-// trip), the conversions are the hardware's (identical to the software
-// rounding for every finite value in range; a row with anything else takes
-// the software rounding), and the group maxima and the scale row go without
-// LDS exchanges and byte stores. Bound by the scattered record writes on large
-// calls, by one row's chain on small ones: 1M BF16 rows 491 -> 427 us (3.7 ->
-// 4.3 TB/s of rows and records), 100,000 rows 55.2 -> 44.2 us, 24 rows x 8
-// layers 29.9 -> 24.9 us; 512k FP32 rows 324 -> 322 us. kStream as in the pack
-// kernel.
+// Native records: one row, RMS-normalised and encoded by a wave. The conversions
+// are the hardware's (identical to the software rounding for every finite value
+// in range; a row with anything else takes the software rounding), and the group
+// maxima and the scale row go without LDS exchanges and byte stores.
 template <bool kBf16, bool kStream>
+__device__ __forceinline__ void native_store_row(const RowRaw& raw, const float (&w)[8], float eps,
+                                                 int64_t slot, int64_t pos, const float* freqs,
+                                                 uint8_t* pool) {
+  const int lane = wave_lane();
+  const bool tail = lane >= kNopeDim / 8;
+  f32x4 fa = {1.f, 0.f, 1.f, 0.f}, fb = fa;
+  if (freqs && tail) {
+    const float* f = freqs + (pos * 4) * (2 * kRopePairs) + 8 * (lane - kNopeDim / 8);
+    fa = *(const f32x4*)f;
+    fb = *(const f32x4*)(f + 4);
+  }
+  float v[8];
+  unpack_raw<kBf16>(raw, v);
+  float p = v[0] * v[0];
+#pragma unroll
+  for (int i = 1; i < 8; ++i) {
+    float sq = v[i] * v[i];
+    p = p + sq;
+  }
+  const float sumsq = wave_tree_sum(p);
+  const float r = inv_rms(sumsq, eps);
+  float y[8];
+  int ai = 0;  // largest magnitude as bits: integer order is float order, non-finite on top
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    y[i] = v[i] * r;
+    y[i] = y[i] * w[i];
+    ai = max(ai, __float_as_int(y[i]) & 0x7fffffff);
+  }
+  ai = max(ai, __builtin_amdgcn_update_dpp(0, ai, kDppXor1, 0xf, 0xf, false));
+  ai = max(ai, __builtin_amdgcn_update_dpp(0, ai, kDppXor2, 0xf, 0xf, false));
+  ai = max(ai, __builtin_amdgcn_update_dpp(0, ai, kDppHalfMirror, 0xf, 0xf, false));
+  // BF16 infinity or beyond anywhere in the row (0x7f7f8000 rounds to it)
+  const bool special = __ballot(ai >= 0x7f7f8000) != 0;
+  uint8_t* page = pool + (slot >> 6) * kNativePageBytes;
+  const int row = (int)(slot & 63);
+  uint8_t* data = page + row * kNativeDataBytes;
+  uint32_t code[2];
+  u32x4 o;
+  int e;
+  if (!special) {
+    bf16x2 nb[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) nb[i] = bf16_pair(y[2 * i], y[2 * i + 1]);
+    e = ue8m0_exponent((float)(__bf16)__int_as_float(ai));
+    const float scale = exp2i(e);
+    s16x2 c01 = {0, 0}, c45 = {0, 0};
+    c01 = fp8_pair<false>(c01, nb[0], scale);
+    c01 = fp8_pair<true>(c01, nb[1], scale);
+    c45 = fp8_pair<false>(c45, nb[2], scale);
+    c45 = fp8_pair<true>(c45, nb[3], scale);
+    code[0] = __builtin_bit_cast(uint32_t, c01);
+    code[1] = __builtin_bit_cast(uint32_t, c45);
+    if (freqs && tail) {
+      const float cs[8] = {fa[0], fa[1], fa[2], fa[3], fb[0], fb[1], fb[2], fb[3]};
+      float nf[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) nf[i] = (float)(__bf16)y[i];
+      rope4(nf, cs);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) nb[i] = bf16_pair(nf[2 * i], nf[2 * i + 1]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = __builtin_bit_cast(uint32_t, nb[i]);
+  } else {
+    float nf[8], amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      nf[i] = bf16_to_f32(bf16_rne(y[i]));
+      amax = fmaxf(amax, fabsf(nf[i]));
+    }
+    amax = fmaxf(amax, __shfl_xor(amax, 1, 64));
+    amax = fmaxf(amax, __shfl_xor(amax, 2, 64));
+    amax = fmaxf(amax, __shfl_xor(amax, 4, 64));
+    e = ue8m0_exponent(amax);
+    const float inv = exp2i(-e);
+    code[0] = code[1] = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      code[0] |= e4m3_rne(nf[i] * inv) << (8 * i);
+      code[1] |= e4m3_rne(nf[4 + i] * inv) << (8 * i);
+    }
+    if (freqs && tail) {
+      const float cs[8] = {fa[0], fa[1], fa[2], fa[3], fb[0], fb[1], fb[2], fb[3]};
+      rope4(nf, cs);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = bf16_rne(nf[2 * i]) | (bf16_rne(nf[2 * i + 1]) << 16);
+  }
+  // scale row: the seven groups' exponents and a zero byte, one 8-byte store
+  uint32_t lo = 0, hi = 0;
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+    lo |= ((uint32_t)(__builtin_amdgcn_readlane(e, 8 * g) + 127) & 0xffu) << (8 * g);
+#pragma unroll
+  for (int g = 4; g < 7; ++g)
+    hi |= ((uint32_t)(__builtin_amdgcn_readlane(e, 8 * g) + 127) & 0xffu) << (8 * (g - 4));
+  if (!tail) {
+    store8<kStream>(u32x2{code[0], code[1]}, (u32x2*)(data + 8 * lane));
+  } else {
+    u32x4* const dst = (u32x4*)(data + kNopeDim + 16 * (lane - kNopeDim / 8));
+    if constexpr (kStream)
+      __builtin_nontemporal_store(o, dst);
+    else
+      *dst = o;
+  }
+  if (lane == 0)
+    store8<kStream>(u32x2{lo, hi},
+                    (u32x2*)(page + kPageRecords * kNativeDataBytes + row * kScaleBytes));
+}
+
+// A skipped row's data is not read: calls often skip many rows (padding), and
+// with every next row loaded ahead of its slot such calls took up to five times
+// as long (131,072 FP32 rows, a quarter stored, 28.7 us with each row waiting
+// for its slot, 45.2 with every row loaded ahead, 21.7 now; none stored 10.7,
+// 38.7, 4.9).
+//   * kOne, up to kNativeBlocks * kWaves rows: at most one row a wave. Up to
+//     kAheadRows (8 or 16 MB of rows, which the latency hides) the row is
+//     requested beside its slot: 8,192 FP32 rows 7.4 -> 6.2 us all stored, 5.8
+//     -> 5.2 a quarter. Beyond, after it (16,384 FP32 rows 13.5 -> 11.1 us,
+//     requested beside it 11.3; a quarter stored 7.8 -> 6.1, 8.8 beside it).
+//   * otherwise a wave loads the slots and positions of its next 64 rows at once
+//     (one a lane), then only the rows that are stored, each while the one before
+//     it is worked on. 16 workgroups a CU (several rows a wave) instead of 64:
+//     65,536 BF16 rows 26.2 us, 32 with 64 a CU; 131,072 47 and 50.
+//   * kStream (above kStreamRows, streaming accesses as in the pack kernel): 64
+//     workgroups a CU again (1M BF16 rows 380 us, 413 with 16, 383 with 128).
+//     BF16 requests a wave's first row beside the slots (384 -> 380; FP32 gains
+//     nothing).
+// Bound by the scattered record writes on large calls (1M BF16 rows move 1,024 +
+// 584 bytes each: 470 -> 380 us, 3.6 -> 4.4 TB/s), by one row's chain of loads
+// and reductions on small ones.
+constexpr int64_t kAheadRows = 8192;
+constexpr int64_t kNativeBlocks = 256 * 16;
+template <bool kBf16, bool kOne, bool kStream>
 __global__ __launch_bounds__(256) void native_store_kernel(
     const void* __restrict__ x, int64_t stride, const float* __restrict__ weight, float eps,
     const int32_t* __restrict__ slots, const int32_t* __restrict__ position,
@@ -590,145 +719,59 @@ __global__ __launch_bounds__(256) void native_store_kernel(
   const int wave = uniform((int)(threadIdx.x >> 6));
   int64_t rec, end, step;
   wave_rows<kBf16>(per, n, wave, rec, end, step);
-  RowRaw cur{};
-  int32_t cur_slot = -1, cur_pos = 0;
-  if (rec < end) {
-    cur = load_raw<kBf16, kStream>(x, rec, stride, lane);
-    cur_slot = slots[rec];
-    if (freqs) cur_pos = position[rec];
-  }
+  if (rec >= end) return;
+  const bool ahead = kOne ? n <= kAheadRows : kStream && kBf16;
+  RowRaw next{};
+  if (ahead) next = load_raw<kBf16, kStream>(x, rec, stride, lane);
+  auto stored = [&](int32_t slot, int32_t pos) {
+    return slot >= 0 && slot < pool_rows && (!freqs || (pos >= 0 && (int64_t)pos * 4 < freq_rows));
+  };
   float w[8];
+  if constexpr (kOne) {
+    const int32_t slot = slots[rec], pos = freqs ? position[rec] : 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w[i] = weight[8 * lane + i];
+    if (!stored(slot, pos)) return;
+    if (!ahead) next = load_raw<kBf16, kStream>(x, rec, stride, lane);
+    native_store_row<kBf16, kStream>(next, w, eps, slot, pos, freqs, pool);
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < 8; ++i) w[i] = weight[8 * lane + i];
-  for (; rec < end; rec += step) {
-    const RowRaw raw = cur;
-    const int64_t slot = cur_slot, pos = cur_pos;
-    if (rec + step < end) {
-      cur = load_raw<kBf16, kStream>(x, rec + step, stride, lane);
-      cur_slot = slots[rec + step];
-      if (freqs) cur_pos = position[rec + step];
+  for (int64_t batch = rec; batch < end; batch += 64 * step) {
+    const int64_t mine = batch + lane * step;
+    int32_t my_slot = -1, my_pos = 0;
+    if (mine < end) {
+      my_slot = slots[mine];
+      if (freqs) my_pos = position[mine];
     }
-    if (slot < 0 || slot >= pool_rows) continue;
-    if (freqs && (pos < 0 || pos * 4 >= freq_rows)) continue;
-    const bool tail = lane >= kNopeDim / 8;
-    f32x4 fa = {1.f, 0.f, 1.f, 0.f}, fb = fa;
-    if (freqs && tail) {
-      const float* f = freqs + (pos * 4) * (2 * kRopePairs) + 8 * (lane - kNopeDim / 8);
-      fa = *(const f32x4*)f;
-      fb = *(const f32x4*)(f + 4);
+    uint64_t todo = __ballot(stored(my_slot, my_pos));  // bit i: row batch + i * step
+    auto load_first = [&]() {
+      next = load_raw<kBf16, kStream>(x, batch + __builtin_ctzll(todo) * step, stride, lane);
+    };
+    if (todo != 0 && !(ahead && batch == rec && (todo & 1))) load_first();
+    while (todo != 0) {
+      const int at = __builtin_ctzll(todo);
+      const RowRaw raw = next;
+      todo &= todo - 1;
+      if (todo != 0) load_first();
+      native_store_row<kBf16, kStream>(raw, w, eps, __builtin_amdgcn_readlane(my_slot, at),
+                                       __builtin_amdgcn_readlane(my_pos, at), freqs, pool);
     }
-    float v[8];
-    unpack_raw<kBf16>(raw, v);
-    float p = v[0] * v[0];
-#pragma unroll
-    for (int i = 1; i < 8; ++i) {
-      float sq = v[i] * v[i];
-      p = p + sq;
-    }
-    const float sumsq = wave_tree_sum(p);
-    const float r = inv_rms(sumsq, eps);
-    float y[8];
-    int ai = 0;  // largest magnitude as bits: integer order is float order, non-finite on top
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      y[i] = v[i] * r;
-      y[i] = y[i] * w[i];
-      ai = max(ai, __float_as_int(y[i]) & 0x7fffffff);
-    }
-    ai = max(ai, __builtin_amdgcn_update_dpp(0, ai, kDppXor1, 0xf, 0xf, false));
-    ai = max(ai, __builtin_amdgcn_update_dpp(0, ai, kDppXor2, 0xf, 0xf, false));
-    ai = max(ai, __builtin_amdgcn_update_dpp(0, ai, kDppHalfMirror, 0xf, 0xf, false));
-    // BF16 infinity or beyond anywhere in the row (0x7f7f8000 rounds to it)
-    const bool special = __ballot(ai >= 0x7f7f8000) != 0;
-    uint8_t* page = pool + (slot >> 6) * kNativePageBytes;
-    const int row = (int)(slot & 63);
-    uint8_t* data = page + row * kNativeDataBytes;
-    uint32_t code[2];
-    u32x4 o;
-    int e;
-    if (!special) {
-      bf16x2 nb[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) nb[i] = bf16_pair(y[2 * i], y[2 * i + 1]);
-      e = ue8m0_exponent((float)(__bf16)__int_as_float(ai));
-      const float scale = exp2i(e);
-      s16x2 c01 = {0, 0}, c45 = {0, 0};
-      c01 = fp8_pair<false>(c01, nb[0], scale);
-      c01 = fp8_pair<true>(c01, nb[1], scale);
-      c45 = fp8_pair<false>(c45, nb[2], scale);
-      c45 = fp8_pair<true>(c45, nb[3], scale);
-      code[0] = __builtin_bit_cast(uint32_t, c01);
-      code[1] = __builtin_bit_cast(uint32_t, c45);
-      if (freqs && tail) {
-        const float cs[8] = {fa[0], fa[1], fa[2], fa[3], fb[0], fb[1], fb[2], fb[3]};
-        float nf[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) nf[i] = (float)(__bf16)y[i];
-        rope4(nf, cs);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) nb[i] = bf16_pair(nf[2 * i], nf[2 * i + 1]);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = __builtin_bit_cast(uint32_t, nb[i]);
-    } else {
-      float nf[8], amax = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        nf[i] = bf16_to_f32(bf16_rne(y[i]));
-        amax = fmaxf(amax, fabsf(nf[i]));
-      }
-      amax = fmaxf(amax, __shfl_xor(amax, 1, 64));
-      amax = fmaxf(amax, __shfl_xor(amax, 2, 64));
-      amax = fmaxf(amax, __shfl_xor(amax, 4, 64));
-      e = ue8m0_exponent(amax);
-      const float inv = exp2i(-e);
-      code[0] = code[1] = 0;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        code[0] |= e4m3_rne(nf[i] * inv) << (8 * i);
-        code[1] |= e4m3_rne(nf[4 + i] * inv) << (8 * i);
-      }
-      if (freqs && tail) {
-        const float cs[8] = {fa[0], fa[1], fa[2], fa[3], fb[0], fb[1], fb[2], fb[3]};
-        rope4(nf, cs);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = bf16_rne(nf[2 * i]) | (bf16_rne(nf[2 * i + 1]) << 16);
-    }
-    // scale row: the seven groups' exponents and a zero byte, one 8-byte store
-    uint32_t lo = 0, hi = 0;
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-      lo |= ((uint32_t)(__builtin_amdgcn_readlane(e, 8 * g) + 127) & 0xffu) << (8 * g);
-#pragma unroll
-    for (int g = 4; g < 7; ++g)
-      hi |= ((uint32_t)(__builtin_amdgcn_readlane(e, 8 * g) + 127) & 0xffu) << (8 * (g - 4));
-    if (!tail) {
-      store8<kStream>(u32x2{code[0], code[1]}, (u32x2*)(data + 8 * lane));
-    } else {
-      u32x4* const dst = (u32x4*)(data + kNopeDim + 16 * (lane - kNopeDim / 8));
-      if constexpr (kStream)
-        __builtin_nontemporal_store(o, dst);
-      else
-        *dst = o;
-    }
-    if (lane == 0)
-      store8<kStream>(u32x2{lo, hi},
-                      (u32x2*)(page + kPageRecords * kNativeDataBytes + row * kScaleBytes));
   }
 }
 
-int grid_for(int64_t n) {
+// 256 CUs x 64 blocks (256 waves per CU over the launch): measured on the
+// 1M-row bulk pack against 32, 128 and 256 blocks per CU, this one is fastest
+constexpr int64_t kMaxBlocks = 256 * 64;
+int grid_for(int64_t n, int64_t cap = kMaxBlocks) {
   int64_t blocks = (n + kWaves - 1) / kWaves;
-  // 256 CUs x 64 blocks (256 waves per CU over the launch): measured on the
-  // 1M-row bulk pack against 32, 128 and 256 blocks per CU, this one is fastest
-  const int64_t cap = 256 * 64;
   return (int)(blocks < cap ? blocks : cap);
 }
 
 // BF16 rows go in runs, FP32 rows (0) at the grid stride.
-int64_t rows_per_wave(bool bf16, int64_t n) {
-  const int64_t waves = (int64_t)grid_for(n) * kWaves;
+int64_t rows_per_wave(bool bf16, int64_t n, int64_t cap = kMaxBlocks) {
+  const int64_t waves = (int64_t)grid_for(n, cap) * kWaves;
   return bf16 ? (n + waves - 1) / waves : 0;
 }
 
@@ -857,12 +900,16 @@ extern "C" int rm_native_store_rows(const void* x, int x_dtype, int64_t x_row_st
     return RM_ERR_ALIGN;
   hipStream_t s = (hipStream_t)stream;
   const int64_t rows = pool_pages * kPageRecords;
-  const bool stream_rows = n > kStreamRows;
-  const auto kern = x_dtype == RM_BF16
-                        ? (stream_rows ? native_store_kernel<true, true> : native_store_kernel<true, false>)
-                        : (stream_rows ? native_store_kernel<false, true> : native_store_kernel<false, false>);
-  hipLaunchKernelGGL(kern, dim3(grid_for(n)), dim3(256), 0, s, x, x_row_stride, weight, eps,
-                     dst_slot, position, freqs, freq_rows, n,
-                     rows_per_wave(x_dtype == RM_BF16, n), pool, rows);
+  const bool bf16 = x_dtype == RM_BF16;
+  const int64_t cap = n > kStreamRows ? kMaxBlocks : kNativeBlocks;
+  const auto kern =
+      n > kStreamRows
+          ? (bf16 ? native_store_kernel<true, false, true> : native_store_kernel<false, false, true>)
+      : n > kNativeBlocks * kWaves
+          ? (bf16 ? native_store_kernel<true, false, false> : native_store_kernel<false, false, false>)
+          : (bf16 ? native_store_kernel<true, true, false> : native_store_kernel<false, true, false>);
+  hipLaunchKernelGGL(kern, dim3(grid_for(n, cap)), dim3(256), 0, s, x, x_row_stride, weight, eps,
+                     dst_slot, position, freqs, freq_rows, n, rows_per_wave(bf16, n, cap), pool,
+                     rows);
   return hipGetLastError() == hipSuccess ? RM_OK : RM_ERR_LAUNCH;
 }

@@ -878,3 +878,58 @@ def test_native_store_sizes_and_non_finite_rows(n, dtype):
                 a[s // 64, s % 64 * 576:s % 64 * 576 + 576] = 0
                 a[s // 64, 36864 + s % 64 * 8:36864 + s % 64 * 8 + 8] = 0
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [8192, 8193, 16384, 16385, 70000, 140000])
+def test_native_store_skipped_rows(n, dtype):
+    """Calls of one row a wave with and without the row requested beside its
+    slot (8,192 and 8,193 rows), several rows a wave (16,385 on) and the
+    streaming form: no row stored, only the first, only the last, runs of
+    skipped rows (some longer than a wave's share), slots and positions out of
+    range. Byte for byte the oracle's, nothing else written."""
+    banner(f"native store skipped rows {n} {dtype}")
+    x = syn.latents(n, seed=83).to(dtype)
+    pages = (n + 63) // 64
+    rng = np.random.default_rng(n)
+    freqs = syn.rope_freqs(4000)
+    keep = np.zeros((5, n), bool)
+    keep[1, 0] = keep[2, -1] = True
+    keep[3] = np.repeat(rng.random(n // 100 + 1) < 0.5, 100)[:n]
+    keep[4] = rng.random(n) < 0.3
+    for k in keep[:5 if n < 50000 else 4]:
+        slots = rng.permutation(pages * 64)[:n].astype(np.int32)
+        slots[~k] = np.resize(np.array([-1, pages * 64], np.int32), n)[~k]
+        pos = np.arange(n, dtype=np.int32) % 1000
+        pos[::41] = np.resize(np.array([-1, 1000], np.int32), pos[::41].size)
+        if k.sum() == 1:
+            pos[k] = 7
+        pool = remnant.LatentPool(pages, fmt="native", device=DEV)
+        pool.buffer.fill_(0x5A)
+        remnant.native_store_rows(x.to(DEV), torch.ones(512, device=DEV), 1e-6,
+                                  torch.from_numpy(slots).to(DEV), torch.from_numpy(pos).to(DEV),
+                                  freqs.to(DEV), pool)
+        ref = np.full((pages, 37376), 0x5A, np.uint8)
+        oracle.native_pack_rows_paged(x.float().numpy(), np.ones(512, np.float32), 1e-6, slots,
+                                      pos, torch.view_as_real(freqs).numpy(), ref)
+        assert np.array_equal(pool.layer().cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_native_store_more_than_64_rows_a_wave(dtype):
+    """4,194,374 rows in one call (65 rows a wave: two batches of slots) store
+    the same bytes as calls of 100,000 rows."""
+    banner(f"native store 4M rows {dtype}")
+    n = 64 * 65536 + 70
+    g = torch.Generator(device=DEV).manual_seed(84)
+    x = torch.randn(n, 512, device=DEV, generator=g, dtype=dtype)
+    slots = torch.randperm(n, device=DEV, generator=g).to(torch.int32)
+    slots[torch.rand(n, device=DEV, generator=g) < 0.2] = -1
+    w = torch.ones(512, device=DEV)
+    pools = [remnant.LatentPool((n + 63) // 64, fmt="native", device=DEV) for _ in range(2)]
+    remnant.native_store_rows(x, w, 1e-6, slots, None, None, pools[0])
+    for i in range(0, n, 100000):
+        remnant.native_store_rows(x[i:i + 100000], w, 1e-6, slots[i:i + 100000], None, None,
+                                  pools[1])
+    torch.cuda.synchronize()
+    assert torch.equal(pools[0].buffer, pools[1].buffer) and pools[0].buffer.any()
