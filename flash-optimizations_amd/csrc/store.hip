@@ -654,8 +654,9 @@ __device__ __forceinline__ void native_store_row(const RowRaw& raw, const float 
     code[0] = code[1] = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      code[0] |= e4m3_rne(nf[i] * inv) << (8 * i);
-      code[1] |= e4m3_rne(nf[4 + i] * inv) << (8 * i);
+      // (an infinity's code is past E4M3: its low byte, as a byte store of it)
+      code[0] |= (e4m3_rne(nf[i] * inv) & 0xffu) << (8 * i);
+      code[1] |= (e4m3_rne(nf[4 + i] * inv) & 0xffu) << (8 * i);
     }
     if (freqs && tail) {
       const float cs[8] = {fa[0], fa[1], fa[2], fa[3], fb[0], fb[1], fb[2], fb[3]};

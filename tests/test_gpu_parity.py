@@ -933,3 +933,40 @@ def test_native_store_more_than_64_rows_a_wave(dtype):
                                   pools[1])
     torch.cuda.synchronize()
     assert torch.equal(pools[0].buffer, pools[1].buffer) and pools[0].buffer.any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_native_store_rows_that_overflow_bf16(dtype):
+    """Finite rows whose normalised values pass the BF16 (and FP32) range under
+    large weights, beside rows that stay finite with scales of up to 2^119: every
+    byte as the oracle writes it, an infinity's code not touching its
+    neighbours' bytes."""
+    banner(f"native store overflow {dtype}")
+    n = 200
+    x = syn.latents(n, seed=79).to(dtype)
+    w = np.ones(512, np.float32)
+    w[5::7] = 2e38  # every 64-coordinate group and the tail
+    pos = np.arange(n, dtype=np.int32)
+    slots = np.random.default_rng(79).permutation(256)[:n].astype(np.int32)
+    freqs = syn.rope_freqs(4 * n)
+    for f in (None, freqs):  # (rotated tails, and tails as stored: their infinities stay)
+        pool = remnant.LatentPool(4, fmt="native", device=DEV)
+        remnant.native_store_rows(x.to(DEV), torch.from_numpy(w).to(DEV), 1e-6,
+                                  torch.from_numpy(slots).to(DEV), torch.from_numpy(pos).to(DEV),
+                                  None if f is None else f.to(DEV), pool)
+        ref = np.zeros((4, 37376), np.uint8)
+        oracle.native_pack_rows_paged(x.float().numpy(), w, 1e-6, slots, pos,
+                                      None if f is None else torch.view_as_real(f).numpy(), ref)
+        got = pool.layer().cpu().numpy()
+        tails = [p[:, :36864].reshape(4, 64, 576)[..., 448:].copy().view(np.uint16)
+                 for p in (got, ref)]
+        inf = np.isinf((tails[1].astype(np.uint32) << 16).view(np.float32))
+        assert f is not None or inf.any()
+        nan = np.isnan((tails[1].astype(np.uint32) << 16).view(np.float32))
+        # (inf - inf in a rotation: the NaN's sign and payload are the machine's)
+        assert np.array_equal(tails[0][~nan], tails[1][~nan])
+        assert np.isnan((tails[0][nan].astype(np.uint32) << 16).view(np.float32)).all()
+        for p in (got, ref):
+            p[:, :36864].reshape(4, 64, 576)[..., 448:] = 0
+        bad = np.nonzero(got != ref)
+        assert bad[0].size == 0, f"{bad[0].size} bytes differ, first {[int(b[0]) for b in bad]}"
