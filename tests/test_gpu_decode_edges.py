@@ -343,22 +343,25 @@ def test_pack_fp32_full_precision_threshold_mantissas_and_ties():
 
 # ---- long splits: a split's record table refilled while it streams ------------------------
 
+@pytest.mark.parametrize("topk", [1504, 2208])
 @pytest.mark.parametrize("packed", [True, False], ids=["direct", "native"])
-def test_decode_long_splits_refilled_table_and_second_pass(packed):
+def test_decode_long_splits_refilled_table_and_second_pass(packed, topk):
     """128 requests x 2 query tokens x 16 heads (256 token x 16-head blocks, so
-    one split per token) at top-k 1504: each split streams 47 stages of 32
-    records, far past the 512 table entries a workgroup holds, so the entries
-    are refilled ring-wise as the split streams. Lengths 1504, 1000, 513, 512,
-    31 and 0 end the split inside, at and before the table's first wrap; q is
-    scaled so later tiles exceed the first tile's max and the split runs a
-    second pass over a rebuilt table. Every row is checked against the oracle."""
-    banner(f"decode long splits packed={packed}")
-    ctx = syn.log_uniform_contexts(128, 6400, 12000, 481)
-    topk = 1504
+    one split per token) at top-k 1504 and 2208: each split streams 47 or 69
+    stages of 32 records. Native's 512 table entries are refilled ring-wise as
+    the split streams, at both; Packed's table holds 2,048 records and is
+    refilled at 2208. Lengths down to 0 end the split inside, at and before the
+    table's first wrap; q is scaled so later tiles exceed the first tile's max
+    and the split runs a second pass over a rebuilt table. Every row is checked
+    against the oracle."""
+    banner(f"decode long splits packed={packed} topk={topk}")
+    ctx = syn.log_uniform_contexts(128, 6400 if topk == 1504 else 8900, 12000, 481)
     c = build_decode_case(ctx, q_len=2, heads=16, topk=topk, seed=481, packed=packed)
     assert remnant.get_decode_metadata(256, 16, topk)[0] == 1
     lens = c["lens"].reshape(-1)
     lens[1:6] = [1000, 513, 512, 31, 0]
+    if topk > 2048:
+        lens[6:9] = [2049, 2048, 2047]
     c["q"] = (c["q"].float() * 300).to(torch.bfloat16)
     out, lse = run_decode(c)
     ref, ref_lse = oracle_decode(c)

@@ -170,20 +170,23 @@ def test_decode_position_mode_per_row_at_realistic_logit_spread(shape):
     assert np.abs(out - out_t).max() <= OUT_TOL
 
 
+@pytest.mark.parametrize("topk", [1504, 2208])
 @pytest.mark.parametrize("rope", ["table", "positions"])
 @pytest.mark.parametrize("swa", [False, True], ids=["c4", "c4+window"])
-def test_decode_long_splits_on_plane_buffers(rope, swa):
-    """Long splits (256 tokens x 16 heads, top-k 1504: one split per token
-    streaming 47 stages, its record table refilled ring-wise) read from plane
-    buffers, with and without window rows: the same bits as the contiguous
-    pool, and every row within the bar of the oracle."""
-    banner(f"decode long splits planes rope={rope} swa={swa}")
-    ctx = syn.log_uniform_contexts(128, 6400, 12000, 631)
-    topk = 1504
+def test_decode_long_splits_on_plane_buffers(rope, swa, topk):
+    """Long splits (256 tokens x 16 heads, one split per token: top-k 1504
+    streams 47 stages from a table of all its records, 2208 streams 69 from a
+    table of 512 slots refilled ring-wise) read from plane buffers, with and
+    without window rows: the same bits as the contiguous pool, and every row
+    within the bar of the oracle."""
+    banner(f"decode long splits planes rope={rope} swa={swa} topk={topk}")
+    ctx = syn.log_uniform_contexts(128, 6400 if topk == 1504 else 8900, 12000, 631)
     c = build_decode_case(ctx, q_len=2, heads=16, topk=topk, seed=631)
     assert remnant.get_decode_metadata(256, 16, topk)[0] == 1
     lens = c["lens"].reshape(-1)
     lens[1:6] = [1000, 513, 512, 31, 0]
+    if topk > 2048:
+        lens[6:9] = [2049, 2048, 2047]
     c["rope"] = rope
     if swa:
         add_swa(c, 64, seed=632)
