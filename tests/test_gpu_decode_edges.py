@@ -355,7 +355,9 @@ def test_decode_long_splits_refilled_table_and_second_pass(packed, topk):
     and the split runs a second pass over a rebuilt table. Every row is checked
     against the oracle."""
     banner(f"decode long splits packed={packed} topk={topk}")
-    ctx = syn.log_uniform_contexts(128, 6400 if topk == 1504 else 8900, 12000, 481)
+    ctx = syn.log_uniform_contexts(128, 6400, 12000, 481)
+    if topk > 2048:  # full lists for 16 tokens (the oracle's time)
+        ctx = syn.log_uniform_contexts(8, 8900, 12000, 481) + [40] * 120
     c = build_decode_case(ctx, q_len=2, heads=16, topk=topk, seed=481, packed=packed)
     assert remnant.get_decode_metadata(256, 16, topk)[0] == 1
     lens = c["lens"].reshape(-1)
@@ -655,8 +657,9 @@ def test_decode_splits_take_consecutive_shares(batch, q_len, heads, topk, splits
     1,024) and refilled (Native at 1,024 and both formats at 2,080 records a
     split, two splits)."""
     banner(f"decode split shares {batch}x{q_len}x{heads} topk={topk} packed={packed}")
-    # contexts beyond the top-k (the lists' lengths are set here)
-    ctx = syn.log_uniform_contexts(batch, 4 * topk + 128, 4 * topk + 800, 541)
+    # (24 tokens at those lengths, the others' lists short: the oracle's time)
+    full = min(batch, -(-24 // q_len))
+    ctx = syn.log_uniform_contexts(full, 4 * topk + 128, 4 * topk + 800, 541) + [40] * (batch - full)
     c = build_decode_case(ctx, q_len=q_len, heads=heads, topk=topk, seed=541, packed=packed)
     lens = c["lens"].reshape(-1)
     stages = (topk + 31) // 32
@@ -665,20 +668,20 @@ def test_decode_splits_take_consecutive_shares(batch, q_len, heads, topk, splits
         if m % splits in (0, 1) or m in (stages - 1, stages):
             edges += [32 * m - 1, 32 * m, 32 * m + 1]
     edges = np.unique(np.minimum(edges, topk))
-    pick = np.linspace(0, edges.size - 1, min(lens.size, edges.size)).astype(int)
-    lens[:] = np.resize(edges[pick], lens.size)
+    pick = np.linspace(0, edges.size - 1, min(full * q_len, edges.size)).astype(int)
+    lens[:full * q_len] = np.resize(edges[pick], full * q_len)
     out, lse, parts = run_split_lse(c, splits)
     ref, ref_lse = oracle_decode(c)
     per_row_check(out, ref, lse, ref_lse)
-    full, sink = c["idx"], c["sink"]
+    lists = c["idx"]
     share = 32 * (-(-(-(-lens // 32)) // splits))
     c["sink"] = None
     for s in range(splits):
         start = np.minimum(s * share, lens)
         count = np.minimum(share, lens - start)
-        idx = full.reshape(lens.size, topk)
+        idx = lists.reshape(lens.size, topk)
         at = np.minimum(start[:, None] + np.arange(max(int(count.max()), 1)), topk - 1)
-        c["idx"] = np.take_along_axis(idx, at, axis=1).reshape(*full.shape[:2], -1).copy()
+        c["idx"] = np.take_along_axis(idx, at, axis=1).reshape(batch, q_len, -1).copy()
         c["lens"] = count.astype(np.int32).reshape(np.shape(c["lens"]))
         part_lse = oracle_decode(c)[1].reshape(lens.size, heads)
         empty = count == 0
