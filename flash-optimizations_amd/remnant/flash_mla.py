@@ -32,10 +32,13 @@ from .packed import (RemnantBuffers, _as_pool, _as_source, _check_cuda, _operand
 def get_decode_metadata(tokens: int, heads: int, topk: int, swa_topk: int = 0) -> tuple[int, int]:
     """(num_splits, workspace_bytes) for a decode of ``tokens`` query tokens
     (``swa_topk`` window rows per token add one partial slot)."""
-    return _plan(tokens, heads, topk, swa_topk)
+    if type(tokens) is int and type(heads) is int and type(topk) is int and type(swa_topk) is int:
+        return _plan(tokens, heads, topk, swa_topk)
+    # (other integers, a 0-d tensor among them, are read on each call)
+    return _plan.__wrapped__(tokens, heads, topk, swa_topk)
 
 
-@functools.lru_cache(maxsize=1024, typed=True)  # a function of the four sizes alone
+@functools.lru_cache(maxsize=1024)  # a function of the four sizes alone
 def _plan(tokens: int, heads: int, topk: int, swa_topk: int) -> tuple[int, int]:
     splits = ctypes.c_int32(0)
     nbytes = ctypes.c_size_t(0)

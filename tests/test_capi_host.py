@@ -129,6 +129,16 @@ def test_decode_split_plan():
         remnant.get_decode_metadata(1, 17, 64)
 
 
+def test_decode_plan_follows_a_tensor_that_changes():
+    """Sizes given as 0-d tensors (or numpy integers) are read on each call: a
+    tensor changed in place gets the plan of its new value."""
+    tokens = torch.tensor(64)
+    assert remnant.get_decode_metadata(tokens, 16, 2048) == remnant.get_decode_metadata(64, 16, 2048)
+    tokens.fill_(1)
+    assert remnant.get_decode_metadata(tokens, 16, 2048) == remnant.get_decode_metadata(1, 16, 2048)
+    assert remnant.get_decode_metadata(1, 16, 2048) != remnant.get_decode_metadata(64, 16, 2048)
+
+
 def test_unpack_gather_host_validation_mirrors_reference():
     pool = torch.zeros((1, config.PACKED_PAGE_BYTES), dtype=torch.uint8)
     index = torch.zeros((1, 1), dtype=torch.int32)
