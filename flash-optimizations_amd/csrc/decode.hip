@@ -208,11 +208,13 @@ constexpr int kPcOddAt = 264;
 __device__ __forceinline__ constexpr int kchunk(int q) { return (q >> 1) * 8 + (q & 1) * kPcOddAt; }
 constexpr int kPcMaxChunk = 512;           // records of a short split; window rows at most
 // Split lengths, each compiled apart: short (at most 512 records), whole
-// (Packed, at most 2,048: a table of that size, built once; it does not fit
-// beside the Native copy ring) and refilled (beyond: a table of 512 slots that
-// a consumer refills as the split streams). The refill and the wave placement
-// and priorities it forbids cost a quarter of a stage: B=128 x next-n 2 at
-// top-k 2048, one split per token, 95.7 us refilled, 78.8 us whole.
+// (Packed, at most 2,048: a table of that size, built once; its 8-byte row
+// addresses do not fit beside the larger Native copy ring) and refilled (beyond:
+// a table of 512 slots that a consumer refills as the split streams). The refill
+// and the wave placement and priorities it forbids cost a quarter of a stage:
+// B=128 x next-n 2 at top-k 2048, one split per token, 95.3 us refilled, 79.5 us
+// whole; 32-head workgroups gain less (32 tokens x 128 heads at top-k 1024 with
+// window rows 67.1 -> 59.3 us).
 enum Len { kShort, kWhole, kRefill };
 constexpr int table_slots(Len l) { return l == kWhole ? 2048 : kPcMaxChunk; }
 constexpr int kBtCache = 1024;             // block-table columns looked up in LDS
@@ -247,8 +249,9 @@ struct PcShared {
   // i % kTab; refilled splits, of more records than that, refill it as they
   // go): pool row address, or (Q address | 1) for an invalid record or a slot
   // past the end (a readable stand-in source, odd so that bit 0 marks it);
-  // Packed: RoPE row address (row 0 of the table for an invalid record, Q
-  // without a table)
+  // Packed, aux_tab: the logical record, whose RoPE row is 256 bytes at that
+  // multiple of 1,024 in the table (0 for an invalid record), or with kPos its
+  // position as a float
   uint64_t row_tab[kTab];
   uint32_t aux_tab[kPacked ? kTab : 1];
   // long splits: the records' top-k entries and block-table entries of the
@@ -404,19 +407,18 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked,
     row_tab[slot] = ok ? (uint64_t)(pg + (r & 63) * (kPlanes ? kCodeBytes : G::kData)) |
                              (kPacked ? 0 : (uint64_t)(r & 63) << 58)
                        : stand_in;
-    // table mode: the record's RoPE row (row 0 of the table for an invalid
-    // record, Q without a table); position mode: the position 4 r as a float
-    // (0 for an invalid record, whose tail is zero)
+    // table mode: the record, for its RoPE row (0 for an invalid one); position
+    // mode: the position 4 r as a float (0 for an invalid record, whose tail is
+    // zero)
     if (kPacked && kPos) aux_tab[slot] = f2u(ok ? (float)(4 * r) : 0.0f);
     else if (kPacked) aux_tab[slot] = ok ? (uint32_t)r : 0u;
   };
   // The table's slots (the first ones of a refilled split), by all waves but
   // the consumers. The list's length, its top-k entries and, for tables of at
   // most kBtCache columns, the request's block-table row are requested side by
-  // side, every load
-  // unconditional (clamped to what is there) so that no wait comes between
-  // two; the row is then looked up in LDS (in the K ring, idle here). The
-  // records' addresses are one memory round trip away from the arguments
+  // side, every load unconditional (clamped to what is there) so that no wait
+  // comes between two; the row is then looked up in LDS (in the K ring, idle
+  // here). The records' addresses are one memory round trip away from the arguments
   // instead of four (length, sequence length, top-k entries, block table).
   // Wider tables look their entries up in memory, one round trip more.
   constexpr int kBuilders = kPcThreads - 64 * kPcConsumers;
@@ -1354,14 +1356,16 @@ __device__ __forceinline__ float lane_of(float x, int l) {
 }
 
 // Merge split partials with the sink, for many rows: one wave per (token,
-// head) row, lane l owning the coordinates stored at 8l..8l+7. The partial loads of up to
-// kWaveBatch splits are issued together with the split LSEs (lane s holds
-// split s), so a row costs one round trip per kWaveBatch splits.
+// head) row, lane l owning the coordinates stored at 8l..8l+7. The partial loads
+// of up to kWaveBatch splits are issued together with the split LSEs (lane s
+// holds split s), so a row costs one round trip per kWaveBatch splits.
 // kWaveBatch is 4 for up to four splits and 8 beyond. Loads past the last split
 // repeat it and are left out of the sum (not added with weight zero: an infinite
-// partial would become a NaN): a branch around each load would make the kernel, which
-// runs once per row, mostly instruction fetch (with the token and head from the
-// grid instead of a division: decode at B=64 0.55 us less a layer, of 33).
+// partial would become a NaN): a branch around each load would make the kernel,
+// which runs once per row, mostly instruction fetch (traced, with the token and
+// head from the grid instead of a division: 64 heads x 16 tokens 4.5 -> 4.1 us, 128
+// heads 5.6 -> 4.9, 16 heads x 64 tokens of four splits 4.6 unchanged; the
+// other combine, one token of 64 splits, 3.9 -> 3.4).
 template <int kWaveBatch>
 __global__ __launch_bounds__(256) void combine_wave_kernel(const float* __restrict__ ws_o,
                                                            const float* __restrict__ ws_lse,

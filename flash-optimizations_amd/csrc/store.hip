@@ -701,7 +701,7 @@ __device__ __forceinline__ void native_store_row(const RowRaw& raw, const float 
 //     (one a lane), then only the rows that are stored, each while the one before
 //     it is worked on. 16 workgroups a CU (several rows a wave) instead of 64:
 //     65,536 BF16 rows 26.2 us, 32 with 64 a CU; 131,072 47 and 50.
-//   * kStream (above kStreamRows, streaming accesses as in the pack kernel): 64
+//   * kStream (above kStreamRows, the pack kernel's limit and accesses): 64
 //     workgroups a CU again (1M BF16 rows 380 us, 413 with 16, 383 with 128).
 //     BF16 requests a wave's first row beside the slots (384 -> 380; FP32 gains
 //     nothing).
