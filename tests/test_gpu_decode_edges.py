@@ -549,6 +549,8 @@ def test_decode_long_split_table_sizes(topk, rope):
     the first one's maximum by more than the slack)."""
     banner(f"decode long-split tables topk={topk} {rope}")
     ctx = syn.log_uniform_contexts(32, 2500, 3000, 503)
+    for b in (0, 1, 20, 31):  # the requests of the long lists
+        ctx[b] = topk + 100
     c = build_decode_case(ctx, q_len=2, heads=128, topk=topk, seed=503, packed=True)
     assert remnant.get_decode_metadata(64, 128, topk)[0] == 1
     c["rope"] = rope
@@ -605,7 +607,7 @@ def test_decode_short_lists_in_whole_tables(heads, rope):
     banner(f"decode short lists in whole tables heads={heads} {rope}")
     batch, q_len = (128, 2) if heads == 16 else (64, 2)
     topk = 2048
-    ctx = syn.log_uniform_contexts(batch, 2100, 2500, 521)
+    ctx = syn.log_uniform_contexts(batch, 4 * topk, 4 * topk + 400, 521)
     c = build_decode_case(ctx, q_len=q_len, heads=heads, topk=topk, seed=521, packed=True)
     assert remnant.get_decode_metadata(batch * q_len, heads, topk)[0] == 1
     c["rope"] = rope
