@@ -375,7 +375,7 @@ __device__ __forceinline__ void decode_pc(const DecodeArgs& a, PcShared<kPacked,
   // but a split then takes its softmax reference from other records and outputs
   // differ in their last bits. Full lists take the same time; 317 of 512 records
   // at 64 heads x B=16, whose three splits then hold 4, 3 and 3 stages instead
-  // of 4, 4 and 2, 64.2 us dealt out and 65.0 us like this, four layers.)
+  // of 4, 4 and 2, 64.2 us dealt out and 64.5-65.0 us like this, four layers.)
   constexpr int kTab = PcShared<kPacked, kLen>::kTab;
   const int k0_full = split * a.chunk;
   int w0 = max(0, k0_full - max(0, kTab - a.chunk));
